@@ -130,6 +130,17 @@ __device__ __forceinline__ float pair_max(float v, int m) {
   return fmaxf(v, pair_val(v, m));
 }
 
+// the largest v of the lane's N neighbours (N = 2 .. 64)
+template <int N>
+__device__ __forceinline__ uint32_t lanes_umax(uint32_t v) {
+#pragma unroll
+  for (int m = 1; m < N; m <<= 1) {
+    const uint32_t o = pair_u(v, m);
+    v = v > o ? v : o;
+  }
+  return v;
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = pair_sum(v, o);

@@ -65,6 +65,10 @@ int arch_from_path(const char* p) {
   return 0;
 }
 
+namespace {
+constexpr uint32_t kDnConvRow = 8192 + 64;  // a token's q, k, v, decay and beta (DnBlockArgs::conv_out)
+}  // namespace
+
 std::unique_ptr<Engine> Engine::create(const uint8_t* bytes, size_t len, const EngineConfig& cfg,
                                        std::string* err) {
   std::unique_ptr<Engine> e(new Engine());
@@ -74,11 +78,10 @@ std::unique_ptr<Engine> Engine::create(const uint8_t* bytes, size_t len, const E
 
 Engine::~Engine() {
   if (stream_) (void)hipStreamSynchronize(stream_);
-  for (int hd = 0; hd < 2; ++hd)
-    for (uint32_t m = 0; m <= kMaxBlock; ++m) {
-      if (bgraph_exec_[hd][m]) (void)hipGraphExecDestroy(bgraph_exec_[hd][m]);
-      if (bgraph_[hd][m]) (void)hipGraphDestroy(bgraph_[hd][m]);
-    }
+  for (uint32_t m = 0; m <= kMaxBlock; ++m) {
+    if (bgraph_exec_[m]) (void)hipGraphExecDestroy(bgraph_exec_[m]);
+    if (bgraph_[m]) (void)hipGraphDestroy(bgraph_[m]);
+  }
   if (graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
   if (graph_) (void)hipGraphDestroy(graph_);
   for (void* p : allocs_) (void)hipFree(p);
@@ -289,6 +292,10 @@ bool Engine::init(const uint8_t* b, size_t len, const EngineConfig& cfg, std::st
     std::string why;
     if (!(bk && bk[0] == '0') && !plan_block(&why) && !why.empty()) {
       *err = "block step: " + why;
+      return false;
+    }
+    if (!(bk && bk[0] == '0') && !plan_panel(&why) && !why.empty()) {
+      *err = "panels: " + why;
       return false;
     }
   }
@@ -845,10 +852,15 @@ void Engine::record_step(hipStream_t st) {
     mark(3);
     enqueue_gemv(dn, hid, 1, GemvMode::Accum, d_mlp_, I, nullptr, st);
   }
+  mark(4);
+  enqueue_head(d_hidden_, st);
+}
+
+// the final norm, LM head and argmax of one hidden row, and the next step's state
+void Engine::enqueue_head(const float* hidden, hipStream_t st) {
   const ProjPlan* lm[1] = {&lm_head_};
   float* lg[1] = {d_logits_};
-  mark(4);
-  const uint32_t n_partials = enqueue_gemv(lm, lg, 1, GemvMode::Logits, d_hidden_, D, d_gamma_final_, st);
+  const uint32_t n_partials = enqueue_gemv(lm, lg, 1, GemvMode::Logits, hidden, uint32_t(arch_.hidden_dim), d_gamma_final_, st);
   FinishArgs f{d_state_, d_prompt_, d_partials_, n_partials, d_logits_, d_result_, d_out_tokens_, embed_args(),
                embed_fused_ ? 1u : 0u};
   launch_finish(f, st);
@@ -927,6 +939,7 @@ int Engine::sync() { return hipStreamSynchronize(stream_) == hipSuccess ? 0 : -3
 int Engine::forward_tokens(const uint32_t* toks, size_t n, ForwardResult* out) {
   if (n == 0 || !toks) return -1;
   if (n > cfg_.max_seq_len) return -2;
+  if (panel_ok_ && n >= 2) return prompt_forward(toks, n, out);  // (one position: the decode step's kernels are faster)
   if (hipMemcpyAsync(d_prompt_, toks, n * 4, hipMemcpyHostToDevice, stream_) != hipSuccess) return -3;
   if (set_state(StepState{toks[0], 0, uint32_t(n), 0})) return -3;
   if (launch_steps(n - 1)) return -3;
@@ -1070,7 +1083,7 @@ bool Engine::plan_block(std::string* err) {
     d_bhx1_ = fa(kMaxBlock * 4096);
     d_bhx2_ = fa(kMaxBlock * 1024);
     d_bhx3_ = fa(kMaxBlock * 32);
-    d_bhconv_ = fa(kMaxBlock * 8192);
+    d_bhconv_ = fa(kMaxBlock * kDnConvRow);
     if (!d_bhx0_ || !d_bhx1_ || !d_bhx2_ || !d_bhx3_ || !d_bhconv_) {
       *err = "allocation";
       return false;
@@ -1223,9 +1236,8 @@ uint32_t Engine::enqueue_block_gemv(const ProjPlan* const* parts, float* const* 
   return launch_block_gemv(b, st);
 }
 
-int Engine::block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t* out_argmax, ForwardResult* last,
-                          bool head) {
-  if (!block_ok_ || !tokens || m == 0 || m > kMaxBlock || (!head && (out_argmax || last))) return -1;
+int Engine::block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t* out_argmax, ForwardResult* last) {
+  if (!block_ok_ || !tokens || m == 0 || m > kMaxBlock) return -1;
   if (pos + m > cfg_.max_seq_len) return -2;
   const uint64_t t0 = now_ns();
   const uint32_t mm = uint32_t(m);
@@ -1236,10 +1248,9 @@ int Engine::block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t
       hipMemcpyAsync(d_bstate_, h_bstate_, sizeof(StepState), hipMemcpyHostToDevice, st) != hipSuccess)
     return -3;
   if (cfg_.hybrid && pos == 0) reset_hybrid_state(st);  // a new sequence (outside the graph)
-  bhead_ = head;
-  if (use_graph_) {  // one captured graph per (head, token count), captured on first use
-    hipGraph_t& g = bgraph_[head ? 1 : 0][m];
-    hipGraphExec_t& ge = bgraph_exec_[head ? 1 : 0][m];
+  if (use_graph_) {  // one captured graph per token count, captured on first use
+    hipGraph_t& g = bgraph_[m];
+    hipGraphExec_t& ge = bgraph_exec_[m];
     if (!ge) {
       if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) != hipSuccess) return -3;
       record_block(mm, st);
@@ -1259,7 +1270,6 @@ int Engine::block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t
       return -3;
     }
   }
-  if (!head) return hipStreamSynchronize(st) == hipSuccess ? 0 : -3;
   if (hipMemcpyAsync(h_bout_, d_bout_, m * 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
       hipMemcpyAsync(h_result_, d_result_, sizeof(StepResult), hipMemcpyDeviceToHost, st) != hipSuccess)
     return -3;
@@ -1307,12 +1317,75 @@ void Engine::record_block(uint32_t mm, hipStream_t st) {
     const ProjPlan* dn[1] = {&L.down};
     n_ss = enqueue_block_gemv(dn, hid, 1, GemvMode::Accum, d_bmlp_, I, nullptr, 0, mm, l, st);
   }
-  if (!bhead_) return;  // (a prefill block before the last: its logits are not read)
   const ProjPlan* lm[1] = {&lm_head_};
   float* lg[1] = {d_blog_};
   const uint32_t eb = enqueue_block_gemv(lm, lg, 1, GemvMode::Logits, d_bx_, D, d_gamma_final_, n_ss, mm, 0, st);
   launch_block_finish(BlockFinishArgs{d_bpartials_, eb, mm, d_blog_, V, btab_.ss, d_bout_, d_result_}, st);
   (void)hipMemcpyAsync(d_logits_, d_blog_ + size_t(mm - 1) * V, size_t(V) * 4, hipMemcpyDeviceToDevice, st);
+}
+
+// the hybrid's q / k norm, rotary and KV append launch over m tokens (state: the first one's position)
+HybQkArgs Engine::hyb_qk_args(size_t l, const StepState* state, const float* qg, const float* k, const float* v,
+                              float* q_out, const uint32_t* brk, uint32_t m) const {
+  const RopeArgs kv = rope_args(l);
+  HybQkArgs q{};
+  q.state = state;
+  q.qg = qg;
+  q.k = k;
+  q.v = v;
+  q.q_norm = hyb_[l].q_norm;
+  q.k_norm = hyb_[l].k_norm;
+  q.rope_cos = d_rope_cos_;
+  q.rope_sin = d_rope_sin_;
+  q.q_out = q_out;
+  q.k_cache = kv.k_cache;
+  q.v_cache = kv.v_cache;
+  q.H = uint32_t(arch_.num_attn_heads);
+  q.KV = uint32_t(arch_.num_kv_heads);
+  q.hd = uint32_t(arch_.head_dim);
+  q.rot = rope_dim_;
+  q.max_seq = kv.max_seq;
+  q.kv_f16 = kv.kv_f16;
+  q.rope_rows = uint32_t(cfg_.max_seq_len);
+  q.eps = arch_.rms_eps;
+  q.m = m;
+  q.qg_stride = 8192;
+  q.kv_stride = 1024;
+  q.q_stride = q.H * q.hd;
+  q.brk = brk;
+  return q;
+}
+
+// the DeltaNet launches over m tokens (x0 .. x3: the in-projections' outputs as d_hx0_ .. d_hx3_)
+DnBlockArgs Engine::dn_block_args(size_t l, const float* x0, const float* x1, const float* x2, const float* x3,
+                                  float* conv, float* out, const uint32_t* brk, uint32_t m) const {
+  DnBlockArgs dn{};
+  dn.x = x0;
+  dn.w = hyb_[l].conv_w;
+  dn.conv_state = d_conv_state_ + size_t(hyb_[l].lin) * 8192 * 3;
+  dn.conv_out = conv;
+  dn.channels = 8192;
+  dn.taps = 4;
+  dn.conv_stride = kDnConvRow;
+  dn.x_stride = 8192;
+  dn.a = x2;
+  dn.b = hyb_[l].has_ab ? x2 + 32 : x3;
+  dn.ab_stride = hyb_[l].has_ab ? 64 : 32;
+  dn.A_log = hyb_[l].A_log;
+  dn.dt_bias = hyb_[l].dt_bias;
+  dn.z = x1;
+  dn.z_stride = 4096;
+  dn.norm_w = hyb_[l].lin_norm;
+  dn.state = d_rec_state_ + size_t(hyb_[l].lin) * 32 * 128 * 128;
+  dn.out = out;
+  dn.out_stride = 4096;
+  dn.n_v_heads = 32;
+  dn.n_k_heads = 16;
+  dn.head_dim = 128;
+  dn.m = m;
+  dn.eps = arch_.rms_eps;
+  dn.brk = brk;
+  return dn;
 }
 
 // The hybrid model's block step: record_step_hybrid's layers for m tokens, every weight read once
@@ -1321,7 +1394,6 @@ void Engine::record_block(uint32_t mm, hipStream_t st) {
 // token (k_hyb_qk over the tokens) and the multi-query decode attention.
 void Engine::record_block_hybrid(uint32_t mm, hipStream_t st) {
   const uint32_t D = uint32_t(arch_.hidden_dim), I = uint32_t(arch_.intermediate_dim), V = uint32_t(arch_.vocab_size);
-  const uint32_t H = uint32_t(arch_.num_attn_heads), KV = uint32_t(arch_.num_kv_heads), hd = uint32_t(arch_.head_dim);
   const uint32_t store[3] = {kRoleStore, kRoleStore, kRoleStore};
   launch_block_embed(embed_args(), d_btok_, mm, d_bx_, d_bss_, d_bbrk_, st);
   uint32_t n_ss = 1;
@@ -1333,33 +1405,7 @@ void Engine::record_block_hybrid(uint32_t mm, hipStream_t st) {
     float* outs[3] = {d_bhx0_, d_bhx1_, d_bhx2_};
     enqueue_block_gemv(in, outs, 3, GemvMode::QkvRope, d_bx_, D, L.gamma_in, n_ss, mm, l, st, store, 32);
     if (Hy.full) {
-      const RopeArgs kv = rope_args(l);
-      HybQkArgs q{};
-      q.state = d_bstate_;
-      q.qg = d_bhx0_;
-      q.k = d_bhx1_;
-      q.v = d_bhx2_;
-      q.q_norm = Hy.q_norm;
-      q.k_norm = Hy.k_norm;
-      q.rope_cos = d_rope_cos_;
-      q.rope_sin = d_rope_sin_;
-      q.q_out = d_bq_;
-      q.k_cache = kv.k_cache;
-      q.v_cache = kv.v_cache;
-      q.H = H;
-      q.KV = KV;
-      q.hd = hd;
-      q.rot = rope_dim_;
-      q.max_seq = kv.max_seq;
-      q.kv_f16 = kv.kv_f16;
-      q.rope_rows = uint32_t(cfg_.max_seq_len);
-      q.eps = arch_.rms_eps;
-      q.m = mm;
-      q.qg_stride = 8192;
-      q.kv_stride = 1024;
-      q.q_stride = H * hd;
-      q.brk = d_bbrk_;
-      launch_hyb_qk(q, st);
+      launch_hyb_qk(hyb_qk_args(l, d_bstate_, d_bhx0_, d_bhx1_, d_bhx2_, d_bq_, d_bbrk_, mm), st);
       AttnArgs at = attn_args(l);
       at.state = d_bstate_;
       at.q = d_bq_;
@@ -1375,32 +1421,7 @@ void Engine::record_block_hybrid(uint32_t mm, hipStream_t st) {
         float* outb[1] = {d_bhx3_};
         enqueue_block_gemv(inb, outb, 1, GemvMode::QkvRope, d_bx_, D, L.gamma_in, n_ss, mm, l, st, store, 32);
       }
-      DnBlockArgs dn{};
-      dn.x = d_bhx0_;
-      dn.w = Hy.conv_w;
-      dn.conv_state = d_conv_state_ + size_t(Hy.lin) * 8192 * 3;
-      dn.conv_out = d_bhconv_;
-      dn.channels = 8192;
-      dn.taps = 4;
-      dn.x_stride = 8192;
-      dn.a = d_bhx2_;
-      dn.b = Hy.has_ab ? d_bhx2_ + 32 : d_bhx3_;
-      dn.ab_stride = Hy.has_ab ? 64 : 32;
-      dn.A_log = Hy.A_log;
-      dn.dt_bias = Hy.dt_bias;
-      dn.z = d_bhx1_;
-      dn.z_stride = 4096;
-      dn.norm_w = Hy.lin_norm;
-      dn.state = d_rec_state_ + size_t(Hy.lin) * 32 * 128 * 128;
-      dn.out = d_battn_;
-      dn.out_stride = 4096;
-      dn.n_v_heads = 32;
-      dn.n_k_heads = 16;
-      dn.head_dim = 128;
-      dn.m = mm;
-      dn.eps = arch_.rms_eps;
-      dn.brk = d_bbrk_;
-      launch_dn_block(dn, st);
+      launch_dn_block(dn_block_args(l, d_bhx0_, d_bhx1_, d_bhx2_, d_bhx3_, d_bhconv_, d_battn_, d_bbrk_, mm), st);
     }
     const ProjPlan* o[1] = {&Hy.out};
     n_ss = enqueue_block_gemv(o, hid, 1, GemvMode::Accum, d_battn_, 4096, nullptr, 0, mm, l, st);
@@ -1410,7 +1431,6 @@ void Engine::record_block_hybrid(uint32_t mm, hipStream_t st) {
     const ProjPlan* dnp[1] = {&L.down};
     n_ss = enqueue_block_gemv(dnp, hid, 1, GemvMode::Accum, d_bmlp_, I, nullptr, 0, mm, l, st);
   }
-  if (!bhead_) return;  // (a prefill block before the last: its logits are not read)
   const ProjPlan* lm[1] = {&lm_head_};
   float* lg[1] = {d_blog_};
   const uint32_t eb = enqueue_block_gemv(lm, lg, 1, GemvMode::Logits, d_bx_, D, d_gamma_final_, n_ss, mm, 0, st);
@@ -1418,22 +1438,263 @@ void Engine::record_block_hybrid(uint32_t mm, hipStream_t st) {
   (void)hipMemcpyAsync(d_logits_, d_blog_ + size_t(mm - 1) * V, size_t(V) * 4, hipMemcpyDeviceToDevice, st);
 }
 
+// ---- panels (a prompt's positions, panel.hip) ---------------------------------------------------
+// Returns false with *err empty when the archive has none (a projection that is neither flat 4- /
+// 2-bit tiles, 4-bit 16-row cells nor fp16 raw tiles), false with *err set on an allocation failure.
+bool Engine::plan_panel(std::string* err) {
+  panel_ok_ = false;
+  const size_t D = arch_.hidden_dim, I = arch_.intermediate_dim;
+  const size_t qd = arch_.num_attn_heads * arch_.head_dim, kvd = arch_.num_kv_heads * arch_.head_dim;
+  if (!block_ok_) {  // (plan_block's archives have whole plans here; otherwise fp16 raw matrices)
+    if (cfg_.hybrid || D % 128 || I % 128 || qd != D || kvd % 2) return false;
+    for (const LayerPlan& L : layers_)
+      for (const ProjPlan* p : {&L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down})
+        if (p->kind != WeightKind::Raw16 || p->bf16 || size_t(p->rows) * p->cols > (size_t(1) << 30)) return false;
+  }
+  auto units = [](size_t rows) { return (rows + 15) / 16; };
+  size_t rows_max = std::max({units(qd) + 2 * units(kvd), 2 * units(I), units(D)}) * 16;
+  if (cfg_.hybrid) rows_max = std::max<size_t>(rows_max, 8192 + 4096 + 64);
+  const size_t Cmax = std::max({D, I, qd}), M = kMaxPanel;
+  ppart_floats_ = std::max(2 * rows_max * kPanelRows, size_t(32) << 20);
+  auto fa = [&](size_t n) { return static_cast<float*>(dev_alloc(n * 4)); };
+  d_px_ = fa(M * D);
+  d_pq_ = fa(M * qd);
+  d_pattn_ = fa(M * qd);
+  d_pmlp_ = fa(M * I);
+  d_pxs_ = static_cast<uint4*>(dev_alloc(kPanelRows * Cmax * (block_ok_ ? 4 : 6)));  // (limbs; three fp16 parts)
+  d_pxt_ = fa(kPanelRows * Cmax);
+  d_ppart_ = fa(ppart_floats_);
+  d_pdown_ = fa(M);
+  d_pss_ = fa((D + 15) / 16 * M);
+  d_pmx_ = static_cast<uint32_t*>(dev_alloc((D + 15) / 16 * M * 4));
+  d_pmax_ = static_cast<uint32_t*>(dev_alloc(2 * arch_.num_layers * kPanelMaxSlots * M * 4));
+  d_pbrk_ = static_cast<uint32_t*>(dev_alloc(M * 4));
+  d_pstate_ = static_cast<StepState*>(dev_alloc(sizeof(StepState)));
+  bool ok = d_px_ && d_pq_ && d_pattn_ && d_pmlp_ && d_pxs_ && d_pxt_ && d_ppart_ && d_pdown_ && d_pss_ && d_pmx_ && d_pmax_ &&
+            d_pbrk_ && d_pstate_;
+  if (cfg_.hybrid) {
+    d_phx0_ = fa(M * 8192);
+    d_phx1_ = fa(M * 4096);
+    d_phx2_ = fa(M * 1024);
+    d_phx3_ = fa(M * 32);
+    d_phconv_ = fa(M * kDnConvRow);
+    ok = ok && d_phx0_ && d_phx1_ && d_phx2_ && d_phx3_ && d_phconv_;
+  }
+  if (!ok) {
+    *err = "allocation";
+    return false;
+  }
+  panel_ok_ = true;
+  return true;
+}
+
+uint32_t Engine::enqueue_panel_gemm(const ProjPlan* const* parts, float* const* outs, int n, GemvMode mode,
+                                    const float* x, uint32_t C, const float* gamma, uint32_t n_ss, uint32_t* max_rows,
+                                    const float* gamma_next, uint32_t m, uint32_t pos, size_t layer,
+                                    hipStream_t st, const uint32_t* roles_in, uint32_t pair_dim) {
+  const uint32_t ng = C / 128;
+  const WeightKind kind = parts[0]->kind;
+  const uint32_t bits = kind == WeightKind::Raw16 ? 16u : kind == WeightKind::FlatW2 ? 2u : 4u;
+  PanelGemmArgs g{};
+  PanelEpiArgs e{};
+  const uint32_t roles[3] = {kRoleQ, kRoleK, kRoleV};
+  uint32_t units = 0;
+  bool corr = false;
+  for (int i = 0; i < n; ++i) {
+    const ProjPlan& p = *parts[i];
+    g.base[i] = p.base;
+    g.stride[i] = p.stride;
+    g.wrows[i] = p.wrows ? p.wrows : p.rows;
+    g.unit_begin[i] = units;
+    PanelPart& P = e.part[i];
+    P.rows = p.rows;
+    P.wrows = g.wrows[i];
+    P.unit_begin = units;
+    P.role = mode == GemvMode::QkvRope ? (roles_in ? roles_in[i] : roles[i]) : 0u;
+    P.y = outs[i];
+    P.bias = p.bias;
+    const bool has = bits != 16 && (p.bcorr || p.corr) && p.boff;
+    P.cpack = has ? p.bpack : nullptr;
+    P.coff = has ? p.boff : nullptr;
+    corr = corr || has;
+    units += (p.rows + 15) / 16;
+    e.total += mode == GemvMode::QkvRope ? p.rows / 2 : (i == 0 ? p.rows : 0u);
+  }
+  const uint32_t rows_all = 16 * units;
+  const PanelShape sh = panel_shape(units, ng, m, bits, ppart_floats_);
+  const uint32_t n_tok = sh.ntt * sh.tile;  // (< m + 112: within the buffers' kPanelRows rows)
+  PanelSplitArgs s{};
+  s.x = x;
+  s.gamma = gamma;
+  s.eps = arch_.rms_eps;
+  s.ssp = d_pss_;
+  s.n_ssp = n_ss;
+  s.tokmax = gamma ? d_pmx_ : max_rows;
+  s.n_max = gamma ? n_ss : kPanelMaxSlots;
+  s.xs = d_pxs_;
+  s.xt = corr ? d_pxt_ : nullptr;
+  s.down = d_pdown_;
+  s.C = C;
+  s.m = m;
+  s.n_tok = n_tok;
+  s.tile = sh.tile;
+  s.brk = d_pbrk_;
+  const RopeArgs rope = rope_args(layer);
+  s.chk = mode == GemvMode::QkvRope ? rope.brk_check : 0u;
+  launch_panel_split(s, bits, st);
+  g.n_parts = n;
+  g.ng = ng;
+  g.n_units = units;
+  g.rows_all = rows_all;
+  g.n_tok = n_tok;
+  g.ntt = sh.ntt;
+  g.nrt = sh.nrt;
+  g.ranges = sh.ranges;
+  g.xs = d_pxs_;
+  g.partial = d_ppart_;
+  launch_panel_gemm(g, bits, sh.tile, st);
+  e.n_parts = n;
+  e.m = m;
+  e.n_tok = n_tok;
+  e.ranges = g.ranges;
+  e.rows_all = rows_all;
+  e.partial = d_ppart_;
+  e.xt = d_pxt_;
+  e.down = d_pdown_;
+  e.pos = pos;
+  e.head_dim = pair_dim ? pair_dim : rope.head_dim;
+  e.max_seq = rope.max_seq;
+  e.kv_f16 = rope.kv_f16;
+  e.rope_rows = uint32_t(cfg_.max_seq_len);
+  e.rope_cos = d_rope_cos_;
+  e.rope_sin = d_rope_sin_;
+  e.k_cache = rope.k_cache;
+  e.v_cache = rope.v_cache;
+  e.ssp_out = d_pss_;
+  e.mx_out = d_pmx_;
+  e.gamma_next = gamma_next;
+  e.tokmax_out = max_rows;
+  e.brk = d_pbrk_;
+  launch_panel_epi(e, mode, st);
+  const uint32_t et = panel_epi_tile(e.total, m);
+  return (e.total + et - 1) / et;  // (Accum: the Σy² partials)
+}
+
+void Engine::enqueue_panel(uint32_t token, uint32_t pos, uint32_t m, hipStream_t st) {
+  const uint32_t D = uint32_t(arch_.hidden_dim), I = uint32_t(arch_.intermediate_dim);
+  const uint32_t H = uint32_t(arch_.num_attn_heads), KV = uint32_t(arch_.num_kv_heads), hd = uint32_t(arch_.head_dim);
+  launch_panel_begin(PanelBeginArgs{d_pstate_, token, pos, d_pmax_, uint32_t(2 * arch_.num_layers) * kPanelMaxSlots * kMaxPanel}, st);
+  launch_block_embed(embed_args(), d_prompt_ + pos, m, d_px_, d_pss_, d_pbrk_, st);
+  launch_panel_rowmax(d_px_, layers_[0].gamma_in, D, m, d_pmx_, st);
+  uint32_t n_ss = 1;  // partial sums and maxima of the hidden rows
+  float* hid[1] = {d_px_};
+  for (size_t l = 0; l < arch_.num_layers; ++l) {
+    const LayerPlan& L = layers_[l];
+    uint32_t* max_attn = d_pmax_ + 2 * l * kPanelMaxSlots * kMaxPanel;
+    uint32_t* max_mlp = max_attn + kPanelMaxSlots * kMaxPanel;
+    const RopeArgs kv = rope_args(l);
+    PanelAttnArgs at{};
+    at.q = d_pq_;
+    at.k_cache = kv.k_cache;
+    at.v_cache = kv.v_cache;
+    at.out = d_pattn_;
+    at.tokmax_out = max_attn;
+    at.H = H;
+    at.KV = KV;
+    at.hd = hd;
+    at.max_seq = kv.max_seq;
+    at.kv_f16 = kv.kv_f16;
+    at.pos = pos;
+    at.m = m;
+    at.scale = 1.0f / std::sqrt(float(hd));
+    if (!cfg_.hybrid) {
+      const ProjPlan* qkv[3] = {&L.q, &L.k, &L.v};
+      float* qo[3] = {d_pq_, nullptr, nullptr};
+      enqueue_panel_gemm(qkv, qo, 3, GemvMode::QkvRope, d_px_, D, L.gamma_in, n_ss, nullptr, nullptr, m, pos, l, st);
+      launch_panel_attention(at, st);
+      const ProjPlan* o[1] = {&L.o};
+      n_ss = enqueue_panel_gemm(o, hid, 1, GemvMode::Accum, d_pattn_, D, nullptr, 0, max_attn, L.gamma_post, m, pos, l, st);
+    } else {
+      const HybLayer& Hy = hyb_[l];
+      const uint32_t store[3] = {kRoleStore, kRoleStore, kRoleStore};
+      const bool ab = !Hy.full && Hy.has_ab;
+      const ProjPlan* in[3] = {&Hy.in0, &Hy.in1, ab ? &Hy.ab : &Hy.in2};
+      float* outs[3] = {d_phx0_, d_phx1_, d_phx2_};
+      enqueue_panel_gemm(in, outs, 3, GemvMode::QkvRope, d_px_, D, L.gamma_in, n_ss, nullptr, nullptr, m, pos, l, st,
+                         store, 32);
+      if (Hy.full) {
+        launch_hyb_qk(hyb_qk_args(l, d_pstate_, d_phx0_, d_phx1_, d_phx2_, d_pq_, d_pbrk_, m), st);
+        at.gate = d_phx0_;
+        launch_panel_attention(at, st);
+      } else {
+        if (!ab) {
+          const ProjPlan* inb[1] = {&Hy.in3};
+          float* outb[1] = {d_phx3_};
+          enqueue_panel_gemm(inb, outb, 1, GemvMode::QkvRope, d_px_, D, L.gamma_in, n_ss, nullptr, nullptr, m, pos, l, st,
+                             store, 32);
+        }
+        DnBlockArgs dn = dn_block_args(l, d_phx0_, d_phx1_, d_phx2_, d_phx3_, d_phconv_, d_pattn_, d_pbrk_, m);
+        dn.tokmax = max_attn;
+        launch_dn_block(dn, st);
+      }
+      const ProjPlan* o[1] = {&Hy.out};
+      n_ss = enqueue_panel_gemm(o, hid, 1, GemvMode::Accum, d_pattn_, 4096, nullptr, 0, max_attn, L.gamma_post, m, pos, l, st);
+    }
+    const ProjPlan* gu[2] = {&L.gate, &L.up};
+    float* mlp[2] = {d_pmlp_, d_pmlp_};
+    enqueue_panel_gemm(gu, mlp, 2, GemvMode::SwiGlu, d_px_, D, L.gamma_post, n_ss, max_mlp, nullptr, m, pos, l, st);
+    const ProjPlan* dn[1] = {&L.down};
+    const float* gamma_next = l + 1 < arch_.num_layers ? layers_[l + 1].gamma_in : d_gamma_final_;
+    n_ss = enqueue_panel_gemm(dn, hid, 1, GemvMode::Accum, d_pmlp_, I, nullptr, 0, max_mlp, gamma_next, m, pos, l, st);
+  }
+}
+
+int Engine::prompt_forward(const uint32_t* tokens, size_t n, ForwardResult* out) {
+  const uint64_t t0 = now_ns();
+  hipStream_t st = stream_;
+  if (hipMemcpyAsync(d_prompt_, tokens, n * 4, hipMemcpyHostToDevice, st) != hipSuccess) return -3;
+  if (cfg_.hybrid) reset_hybrid_state(st);  // a new sequence
+  // equal panels
+  const size_t np = (n + kMaxPanel - 1) / kMaxPanel, per = (n + np - 1) / np;
+  size_t m = 0;
+  for (size_t i = 0; i < n; i += per) {
+    m = std::min(per, n - i);
+    enqueue_panel(tokens[i], uint32_t(i), uint32_t(m), st);
+  }
+  // the last position's LM head and argmax as the decode step's: its state at position n - 1, the
+  // next one at the argmax and position n
+  *h_state_ = StepState{tokens[n - 1], uint32_t(n - 1), 0, 0};
+  h_pos_ = n;
+  const float* last = d_px_ + (m - 1) * arch_.hidden_dim;
+  if (hipMemcpyAsync(d_state_, h_state_, sizeof(StepState), hipMemcpyHostToDevice, st) != hipSuccess) return -3;
+  if (!embed_fused_ &&
+      hipMemcpyAsync(d_hidden_, last, arch_.hidden_dim * 4, hipMemcpyDeviceToDevice, st) != hipSuccess)
+    return -3;
+  enqueue_head(last, st);
+  if (hipMemcpyAsync(h_result_, d_result_, sizeof(StepResult), hipMemcpyDeviceToHost, st) != hipSuccess) return -3;
+  if (sync()) return -3;
+  out->argmax_token = h_result_->argmax;
+  out->max_logit = h_result_->max_logit;
+  out->token0_logit = h_result_->token0_logit;
+  out->hidden_norm = h_result_->hidden_norm;
+  out->all_finite = h_result_->all_finite != 0;
+  out->elapsed_ns = now_ns() - t0;
+  return 0;
+}
+
 int Engine::prefill(const uint32_t* tokens, size_t n, ForwardResult* out) {
   if (!tokens || n == 0 || !out) return -1;
   if (n > cfg_.max_seq_len) return -2;
+  if (panel_ok_ && n > kMaxBlock) return prompt_forward(tokens, n, out);  // (a short prompt: the block step's graph)
   if (!block_ok_) {  // no block step for this archive: sequential steps
     const int rc = forward_tokens(tokens, n, out);
     if (rc) return rc;
     h_pos_ = n;
     return 0;
   }
-  uint32_t am[kMaxBlock];
-  for (size_t i = 0; i < n; i += kMaxBlock) {
-    const size_t m = std::min<size_t>(kMaxBlock, n - i);
-    const bool head = i + m == n;  // (only the last block's logits are read)
-    const int rc = block_forward(tokens + i, m, i, head ? am : nullptr, head ? out : nullptr, head);
-    if (rc) return rc;
-  }
+  uint32_t am[kMaxBlock];  // (n <= kMaxBlock: one block step)
+  const int rc = block_forward(tokens, n, 0, am, out);
+  if (rc) return rc;
   // continue greedy decoding from here: the last argmax at position n
   if (set_state(StepState{out->argmax_token, uint32_t(n), 0, 0})) return -3;
   return sync();
@@ -1743,13 +2004,8 @@ void Engine::record_step_hybrid(hipStream_t st) {
     mark(3);
     enqueue_gemv(dn, hid, 1, GemvMode::Accum, d_mlp_, I, nullptr, st);
   }
-  const ProjPlan* lm[1] = {&lm_head_};
-  float* lg[1] = {d_logits_};
   mark(4);
-  const uint32_t n_partials = enqueue_gemv(lm, lg, 1, GemvMode::Logits, d_hidden_, D, d_gamma_final_, st);
-  FinishArgs f{d_state_, d_prompt_, d_partials_, n_partials, d_logits_, d_result_, d_out_tokens_, embed_args(),
-               embed_fused_ ? 1u : 0u};
-  launch_finish(f, st);
+  enqueue_head(d_hidden_, st);
 }
 
 int Engine::launch_stage(int stage, size_t l) {

@@ -155,13 +155,16 @@ class Engine {
   // its result *last.  The decode state is not touched.  0, -1 bad arguments or no block step
   // for this archive, -2 past max_seq_len, -3 device error.  (verify() and prefill() then leave
   // the decode state where the sequential steps would: the last argmax at pos + m.)
-  // head false: no LM head (out_argmax and last must be null; the prefill's blocks before its last)
-  int block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t* out_argmax, ForwardResult* last,
-                    bool head = true);
+  int block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t* out_argmax, ForwardResult* last);
   bool block_ready() const { return block_ok_; }
-  // positions 0..n-1 teacher-forced in blocks of kMaxBlock (prefill); result and logits of
-  // the last position; the decode state is left at (argmax of the last, n)
+  // positions 0..n-1 teacher-forced: one block step up to kMaxBlock positions, panels
+  // (prompt_forward) above; result and logits of the last position; the decode state is left at
+  // (argmax of the last, n)
   int prefill(const uint32_t* tokens, size_t n, ForwardResult* out);
+  // the prompt in panels of up to kMaxPanel positions (plan_panel's archives; prefill and
+  // forward_tokens call it): every weight is read once per panel; result, logits, hidden state and
+  // decode state are left as the sequential steps leave them (the last argmax at position n)
+  int prompt_forward(const uint32_t* tokens, size_t n, ForwardResult* out);
   // enqueue n graph launches continuing from the current device state (no sync); -2 and
   // nothing enqueued when the steps would pass max_seq_len
   int launch_steps(size_t n);
@@ -233,6 +236,21 @@ class Engine {
                               const float* x, uint32_t C, const float* gamma, uint32_t n_ss, uint32_t m,
                               size_t layer, hipStream_t st, const uint32_t* roles = nullptr, uint32_t pair_dim = 0);
   void record_block_hybrid(uint32_t m, hipStream_t st);  // record_block of the hybrid model
+  void enqueue_head(const float* hidden, hipStream_t st);
+  HybQkArgs hyb_qk_args(size_t l, const StepState* state, const float* qg, const float* k, const float* v, float* q_out,
+                        const uint32_t* brk, uint32_t m) const;
+  DnBlockArgs dn_block_args(size_t l, const float* x0, const float* x1, const float* x2, const float* x3, float* conv,
+                            float* out, const uint32_t* brk, uint32_t m) const;
+  bool plan_panel(std::string* err);
+  // m positions pos .. of the prompt (its tokens at d_prompt_ + pos) through every layer
+  void enqueue_panel(uint32_t token, uint32_t pos, uint32_t m, hipStream_t st);
+  // a panel's projections of one input.  gamma: the rows' partial sums and maxima are in d_pss_ and
+  // d_pmx_ (n_ss each), where Accum leaves the updated rows' (of |y * gamma_next|); otherwise max_rows
+  // holds their maxima, where SwiGlu leaves its output's.  roles, pair_dim as enqueue_block_gemv
+  uint32_t enqueue_panel_gemm(const ProjPlan* const* parts, float* const* outs, int n, GemvMode mode, const float* x,
+                              uint32_t C, const float* gamma, uint32_t n_ss, uint32_t* max_rows,
+                              const float* gamma_next, uint32_t m, uint32_t pos, size_t layer, hipStream_t st,
+                              const uint32_t* roles = nullptr, uint32_t pair_dim = 0);
 
  public:
   // run one projection's GEMV on a caller vector (Store mode, bias included): parity hooks
@@ -308,11 +326,19 @@ class Engine {
   float *d_bhx0_ = nullptr, *d_bhx1_ = nullptr, *d_bhx2_ = nullptr, *d_bhx3_ = nullptr, *d_bhconv_ = nullptr;
   BlockTables btab_{};
   ArgmaxPartial* d_bpartials_ = nullptr;
-  // captured block steps, by [with the LM head][token count]; bhead_: the one being recorded has
-  // the LM head (the prefill's blocks before its last have none: their logits are not read)
-  hipGraph_t bgraph_[2][kMaxBlock + 1] = {};
-  hipGraphExec_t bgraph_exec_[2][kMaxBlock + 1] = {};
-  bool bhead_ = true;
+  // captured block steps, by token count
+  hipGraph_t bgraph_[kMaxBlock + 1] = {};
+  hipGraphExec_t bgraph_exec_[kMaxBlock + 1] = {};
+  // the panels (plan_panel): activations of kMaxPanel rows, the GEMM's fp16 input images, partial
+  // sums, per-token scales, maxima [2 per layer][kPanelMaxSlots][kMaxPanel] and break flags
+  bool panel_ok_ = false;
+  float *d_px_ = nullptr, *d_pq_ = nullptr, *d_pattn_ = nullptr, *d_pmlp_ = nullptr, *d_pxt_ = nullptr;
+  float *d_ppart_ = nullptr, *d_pdown_ = nullptr, *d_pss_ = nullptr;
+  float *d_phx0_ = nullptr, *d_phx1_ = nullptr, *d_phx2_ = nullptr, *d_phx3_ = nullptr, *d_phconv_ = nullptr;
+  uint4* d_pxs_ = nullptr;
+  uint32_t *d_pmax_ = nullptr, *d_pmx_ = nullptr, *d_pbrk_ = nullptr;
+  StepState* d_pstate_ = nullptr;
+  size_t ppart_floats_ = 0;
   int probe_stage_ = -1;                 // stage bracketed by events in record_step
   hipEvent_t* probe_events_ = nullptr;
   size_t probe_next_ = 0;

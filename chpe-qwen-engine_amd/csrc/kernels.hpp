@@ -391,8 +391,10 @@ struct DnBlockArgs {
   const float* x;           // conv input [m][x_stride] (channels used)
   const float* w;           // [channels][taps]
   float* conv_state;        // [channels][taps-1]
-  float* conv_out;          // [m][channels]: q [n_k_heads][hd], k, v [n_v_heads][hd] per token
-  uint32_t channels, taps, x_stride;
+  // [m][conv_stride]: q [n_k_heads][hd], k (both normalised), v [n_v_heads][hd], then decay and beta
+  // [n_v_heads] per token
+  float* conv_out;
+  uint32_t channels, taps, x_stride, conv_stride;
   const float *a, *b;       // [m][ab_stride]
   uint32_t ab_stride;
   const float *A_log, *dt_bias;
@@ -405,6 +407,7 @@ struct DnBlockArgs {
   uint32_t n_v_heads, n_k_heads, head_dim, m;
   float eps;
   const uint32_t* brk;      // [m]: token t broke before this layer (its state updates are skipped)
+  uint32_t* tokmax;         // or null: [kPanelMaxSlots][kMaxPanel] maxima of |out|
 };
 void launch_dn_block(const DnBlockArgs& a, hipStream_t stream);
 
@@ -453,6 +456,88 @@ inline uint32_t attn_chunk(uint32_t hd, uint32_t kv) { return attn_chunk_of(hd, 
 // (hd, query heads per kv head) pairs the attention kernels are built for
 bool attention_supported(uint32_t H, uint32_t KV, uint32_t hd);
 constexpr uint32_t kMaxLogitsBlocks = 8192;
+
+// ---- panels: up to kMaxPanel tokens of a prompt at consecutive positions (panel.hip) ------------
+constexpr uint32_t kMaxPanel = 512;
+constexpr uint32_t kPanelRows = kMaxPanel + 112;  // rows of the GEMM's buffers: m in whole tiles of up to 112 tokens
+// Attention and the SwiGLU leave the largest |value| of each row as atomic maxima (of the bits) in
+// kPanelMaxSlots rows of [kMaxPanel] (a workgroup uses one of them: in a single row of 32 tokens to a cache line the 688
+// workgroups of a SwiGLU launch queue on one line, 45 us instead of 6)
+constexpr uint32_t kPanelMaxSlots = 16;
+struct PanelBeginArgs {    // the panel's state and cleared maxima
+  StepState* state;
+  uint32_t token, pos;
+  uint32_t* tokmax;        // [n_max]
+  uint32_t n_max;
+};
+struct PanelSplitArgs {    // a GEMM's input rows as matrix-core operands
+  const float* x;          // [m][C]
+  const float* gamma;      // RMSNorm gains, or null
+  float eps;
+  const float* ssp;        // (gamma) [n_ssp][kMaxPanel]: partial sums of x^2 of the rows
+  uint32_t n_ssp;
+  const uint32_t* tokmax;  // [n_max][kMaxPanel]: partial maxima, as bits, of |x| (gamma: of |x * gamma|) of the rows
+  uint32_t n_max;
+  uint4* xs;               // [token tile][group]: the GEMM's LDS images (k_panel_split)
+  float* xt;               // [C][n_tok] f32, token-minor, or null
+  float* down;             // [m]: the factor from a row's products to its values
+  uint32_t C, m, n_tok, tile;  // n_tok: m rounded up to whole token tiles
+  uint32_t* brk;           // [m] break flags, set by the test chk (RopeArgs::brk_check)
+  uint32_t chk;
+};
+struct PanelGemmArgs {
+  const uint8_t* base[kMaxParts];
+  uint32_t stride[kMaxParts], wrows[kMaxParts], unit_begin[kMaxParts];
+  int n_parts;
+  uint32_t ng, n_units, rows_all;  // groups; 16-row units; 16 * n_units
+  uint32_t n_tok, ntt, nrt, ranges;  // tokens (whole tiles), token tiles, row tiles of 16 units
+  const uint4* xs;
+  float* partial;          // [ranges][rows_all][n_tok]
+};
+struct PanelPart {
+  uint32_t rows, wrows, unit_begin, role;
+  float* y;                // [m][rows]
+  const float* bias;
+  const float2* cpack;     // packed outlier corrections and each row's first entry, or null
+  const uint32_t* coff;
+};
+struct PanelEpiArgs {
+  PanelPart part[kMaxParts];
+  int n_parts;
+  uint32_t m, n_tok, ranges, rows_all, total;  // total: outputs (rows of part 0; RoPE pairs of all parts)
+  const float* partial;
+  const float* xt;
+  const float* down;
+  uint32_t pos, head_dim, max_seq, kv_f16, rope_rows;
+  const float *rope_cos, *rope_sin;
+  void *k_cache, *v_cache;
+  float* ssp_out;          // Accum: [total / panel_epi_tile][kMaxPanel] partial sums of y^2,
+  uint32_t* mx_out;        //   and maxima of |y * gamma_next|
+  const float* gamma_next; //   (the gains of the norm that reads the rows next)
+  uint32_t* tokmax_out;    // SwiGlu: [kPanelMaxSlots][kMaxPanel] maxima of |y|
+  const uint32_t* brk;
+};
+struct PanelAttnArgs {
+  const float* q;          // [m][H][hd]
+  const void *k_cache, *v_cache;  // as AttnArgs
+  float* out;              // [m][H][hd]
+  const float* gate;       // or null: as AttnArgs
+  uint32_t* tokmax_out;    // [kPanelMaxSlots][kMaxPanel] maxima of |out|
+  uint32_t H, KV, hd, max_seq, kv_f16, pos, m;
+  float scale;
+};
+void launch_panel_begin(const PanelBeginArgs& a, hipStream_t stream);
+void launch_panel_rowmax(const float* x, const float* gamma, uint32_t C, uint32_t m, uint32_t* mx_out, hipStream_t stream);
+void launch_panel_split(const PanelSplitArgs& a, uint32_t bits, hipStream_t stream);
+void launch_panel_gemm(const PanelGemmArgs& a, uint32_t bits, uint32_t tile, hipStream_t stream);
+void launch_panel_epi(const PanelEpiArgs& a, GemvMode mode, hipStream_t stream);
+void launch_panel_attention(const PanelAttnArgs& a, hipStream_t stream);
+uint32_t panel_epi_tile(uint32_t total, uint32_t m);  // outputs per epilogue workgroup
+// how a GEMM of n_units units, ng groups and m tokens is cut up (at most max_partials partial sums)
+struct PanelShape {
+  uint32_t tile, ntt, nrt, ranges;  // tokens per tile, token tiles, row tiles, column ranges
+};
+PanelShape panel_shape(uint32_t n_units, uint32_t ng, uint32_t m, uint32_t bits, size_t max_partials);
 
 // Measurement: the next kernel launched by any launcher on this host thread records `start`
 // and `stop` when it begins and ends (hipExtLaunchKernelGGL), then the probe is cleared.

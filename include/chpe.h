@@ -29,7 +29,8 @@ void *chpe_init(const char *archive_path);
 /* chpe_c_api.zig:50-78 `chpe_forward_tokens`: decode positions 0..num_tokens-1.
  * Returns the last argmax, -1 if ctx/tokens is NULL or num_tokens == 0, -2 if num_tokens
  * exceeds the context's max_seq_len, -3 on a device error.  out_logits (optional) receives
- * vocab_size floats of the last step. */
+ * vocab_size floats of the last step.  Two positions and more run in panels where the archive has
+ * them (chpe_prefill); chpe_get_last_elapsed_ns is then the whole call's time. */
 int chpe_forward_tokens(void *ctx, const uint32_t *tokens, size_t num_tokens, float *out_logits);
 
 /* chpe_c_api.zig:80-87 `chpe_get_last_logits`: copies vocab_size floats of the last step;
@@ -79,11 +80,11 @@ int chpe_generate(void *ctx, const uint32_t *prompt, size_t n_prompt, size_t n_g
  * the decode step, bit-identical.  last_* report the final step; chpe_get_last_logits gives
  * its logits.  Returns 0, -1 bad args, -2 pos + m > max_seq_len, -3 device error. */
 int chpe_verify(void *ctx, const uint32_t *drafts, size_t m, size_t pos, uint32_t *out_argmax);
-/* Prefill: positions 0..num_tokens-1 teacher-forced as chpe_forward_tokens, in block steps of
- * up to 32 tokens that read every weight once per block (archives of flat 4- or 2-bit tiles or
- * 4-bit 16-row cells; others:
- * the sequential steps).  Each token's arithmetic is the decode step's up to the order of the
- * float sums; the KV cache holds the same rows.  Leaves the decode state at (the last argmax,
+/* Prefill: positions 0..num_tokens-1 teacher-forced as chpe_forward_tokens: up to 32 positions as
+ * one block step, more in panels of up to 512 positions, each reading every weight once (archives of
+ * flat 4- or 2-bit tiles, 4-bit 16-row cells or fp16 raw tiles; others: the sequential steps).  Each
+ * token's arithmetic is the decode step's up to the order of the float sums; the KV cache holds the
+ * same rows.  Leaves the decode state at (the last argmax,
  * num_tokens).  Returns the last argmax, -1 bad args, -2 too long, -3 device error;
  * out_logits (optional) receives the last position's logits. */
 int chpe_prefill(void *ctx, const uint32_t *tokens, size_t num_tokens, float *out_logits);

@@ -1,0 +1,107 @@
+"""A prompt in panels (chpe_forward_tokens, and chpe_prefill past one block step) against the decode
+steps of an engine that has neither (CHPE_BLOCK=0): the last position's logits and hidden state, and
+the next decode step's logits, which read every cache row and recurrent state the panels left.
+
+Prompt lengths at the edges of the token tiles (32, 64), of the DeltaNet chunk (32) and of the panel
+(512), and odd ones.  The 2-norm bars: with the f32 cache each path is within 1e-5 of the 64-bit
+result (f32 sums over 36 layers; measured 1e-6 to 8e-6), so they differ by less than 2e-5, with as
+much again for the prompt; with the fp16 cache, rows whose f32 value lies within that distance of a
+rounding boundary are stored one fp16 step apart (2^-11 of the value): measured 1e-5 to 2e-4, the
+bars four times that.  An argmax may differ only where the two best logits are closer
+than the bar.  (The 72B archives' panels: test_gpu_models.py, a prompt of 11 against the block step
+and the oracle.)"""
+import os
+
+import numpy as np
+import pytest
+
+import chpe_amd as ca
+from conftest import archive_path
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # archive kind, arch, vocabulary, fp16 cache, prompt lengths, bar
+    (ca.PACK_3B_W4, 0, 151936, False, (2, 32, 33, 64, 65, 129, 512, 513, 577), 4e-5),
+    (ca.PACK_3B_W4, 0, 151936, True, (3, 97, 600), 8e-4),
+    (ca.PACK_3B_FP16_RAW, 0, 151936, False, (2, 31, 33, 64, 100, 515), 4e-5),
+    (ca.PACK_3B_FP16_RAW, 0, 151936, True, (7, 130), 8e-4),
+    (ca.PACK_9B_W4, 3, 248320, True, (2, 3, 4, 32, 33, 65, 100, 513), 8e-4),
+    (ca.PACK_9B_W4, 3, 248320, False, (5, 70), 8e-5),
+    (ca.PACK_9B_W4, 1, 248320, False, (34, 70), 8e-5),
+]
+
+
+def rel(a, b):
+    b = b.astype(np.float64)
+    return float(np.linalg.norm(a.astype(np.float64) - b) / np.linalg.norm(b))
+
+
+def engines(path, arch, rows, kv16, monkeypatch):
+    monkeypatch.setenv("CHPE_BLOCK", "0")
+    steps = ca.Engine(path, arch=arch, max_seq_len=rows, kv_f16=kv16)
+    monkeypatch.delenv("CHPE_BLOCK")
+    return ca.Engine(path, arch=arch, max_seq_len=rows, kv_f16=kv16), steps
+
+
+@pytest.mark.timeout(600)
+@pytest.mark.parametrize("kind,arch,vocab,kv16,lengths,bar", CASES)
+def test_panels_match_decode_steps(kind, arch, vocab, kv16, lengths, bar, monkeypatch):
+    e, steps = engines(archive_path(kind), arch, max(lengths) + 8, kv16, monkeypatch)
+    try:
+        for n in lengths:
+            toks = np.random.default_rng(1000 * kind + n).integers(0, vocab, n).astype(np.uint32)
+            am0, want = steps.forward_tokens(toks, want_logits=True)
+            hid0 = steps.hidden()
+            nxt0 = steps.decode_step(int(toks[0]), n)[1]
+            calls = [e.forward_tokens] + ([e.prefill] if n > 32 else [])
+            for call in calls:
+                am, got = call(toks, want_logits=True)
+                hid = e.hidden()
+                nxt = e.decode_step(int(toks[0]), n)[1]
+                d = (rel(got, want), rel(hid, hid0), rel(nxt, nxt0))
+                print(f"kind {kind} arch {arch} kv16 {kv16} n {n} {call.__name__}: logits {d[0]:.2e} hidden {d[1]:.2e} next {d[2]:.2e}",
+                      flush=True)
+                assert max(d) <= bar
+                if am != am0:
+                    assert want[am0] - want[am] <= bar * np.linalg.norm(want)
+            # the greedy loop goes on from the state the prompt left
+            assert np.array_equal(e.forward_tokens(toks, want_logits=True)[1].view(np.uint32),
+                                  e.forward_tokens(toks, want_logits=True)[1].view(np.uint32))
+    finally:
+        e.close()
+        steps.close()
+
+
+def test_panel_break(w4_archive, monkeypatch):
+    """forwardDecode's non-finite break (StepState::broken) in a panel: an infinite outlier weight
+    in layer 1's down projection stops every token after that layer; the final norm and the LM head
+    see that hidden state, as in the decode steps."""
+    import tempfile
+
+    import oracle as orc
+    from test_gpu_nonfinite import inf_outlier_edit
+    li = orc.layer_info(1, 1)
+    off, b = inf_outlier_edit(w4_archive, li["down_proj"], li["down_tiles"])
+    data = np.fromfile(w4_archive, dtype=np.uint8)
+    data[off:off + 2] = np.frombuffer(b, np.uint8)
+    fd, path = tempfile.mkstemp(suffix=".chpe", prefix="qwen2.5-3b-mod-", dir=os.path.dirname(str(w4_archive)))
+    os.close(fd)
+    data.tofile(path)
+    try:
+        e, steps = engines(path, 0, 64, False, monkeypatch)
+        try:
+            toks = np.random.default_rng(3).integers(0, 151936, 40).astype(np.uint32)
+            am0, want = steps.forward_tokens(toks, want_logits=True)
+            hid0, last0 = steps.hidden(), steps.last()
+            am, got = e.forward_tokens(toks, want_logits=True)
+            hid, last = e.hidden(), e.last()
+            assert not np.isfinite(hid0).all()
+            fin = np.isfinite(hid0)
+            assert np.array_equal(np.isfinite(hid), fin) and rel(hid[fin], hid0[fin]) <= 4e-5
+            assert np.array_equal(np.isnan(got), np.isnan(want)) and am == am0
+            assert last["hidden_norm"] == last0["hidden_norm"] == np.inf
+        finally:
+            e.close()
+            steps.close()
+    finally:
+        os.unlink(path)
