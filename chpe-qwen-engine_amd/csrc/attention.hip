@@ -43,7 +43,15 @@ __device__ __forceinline__ AttnArgs attn_query(AttnArgs a) {
   return a;
 }
 
-template <int HD, int GQ, typename KT, int LPP, int NW>
+// The position of the (first) query: the device state's, or, for a launch whose caller knows it
+// (FIX), an argument -- as a compile-time choice, so that the state's load stays the first one.
+template <bool FIX>
+__device__ __forceinline__ uint32_t attn_pos(const AttnArgs& a) {
+  if constexpr (FIX) return a.pos;
+  else return a.state->pos;
+}
+
+template <int HD, int GQ, typename KT, int LPP, int NW, bool FIX>
 __global__ void __launch_bounds__(NW * 64) k_attn_chunk(AttnArgs a0) {
   const AttnArgs a = attn_query(a0);
   using E = KvElem<KT>;
@@ -54,7 +62,7 @@ __global__ void __launch_bounds__(NW * 64) k_attn_chunk(AttnArgs a0) {
   constexpr int DPL = HD / 64;              // V dims per lane
   constexpr int VW = DPL * E::kBytes / 4;   // 32-bit words of a lane's V dims (1, 2 or 4)
   static_assert(KW % 4 == 0 && VW >= 1, "");
-  const uint32_t pos = a.state->pos + blockIdx.z, ctx = pos + 1;
+  const uint32_t pos = attn_pos<FIX>(a) + blockIdx.z, ctx = pos + 1;
   const uint32_t c = blockIdx.x, kvh = blockIdx.y;
   if (c * CH >= ctx) return;  // the whole workgroup
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -235,7 +243,7 @@ __device__ __forceinline__ h4_t f16_part(float a, float b, float c, float d, boo
   return rem ? r : h;
 }
 
-template <int HD, int GQ, int NW, int T, int QZ>
+template <int HD, int GQ, int NW, int T, int QZ, bool FIX>
 __global__ void __launch_bounds__(NW * 64) k_attn_mfma(AttnArgs a) {
   constexpr int KD = HD / 4;   // K dims per lane
   constexpr int KS = HD / 16;  // k-steps of the score product
@@ -247,7 +255,7 @@ __global__ void __launch_bounds__(NW * 64) k_attn_mfma(AttnArgs a) {
   // for only after the loads below are issued
   const uint32_t nz = a.nq > 1 ? a.nq : 1u, z0 = blockIdx.z * QZ;
   const uint32_t z1 = QZ == 1 ? z0 + 1 : (z0 + QZ < nz ? z0 + QZ : nz);  // (QZ = 1: grid.z = nz)
-  const uint32_t pos0 = a.state->pos;
+  const uint32_t pos0 = attn_pos<FIX>(a);
   const size_t qrows = size_t(a.H) * HD;  // one query's rows of q / out
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int G = lane >> 4, n = lane & 15, h = n & 7;  // h: the query head of column / row n
@@ -558,7 +566,7 @@ __global__ void __launch_bounds__(256) k_attn_mq(AttnArgs a) {
 // context are masked), the waves' sums meet in LDS in wave order.  Every wave forms the chunk
 // weights exp(m_c - M) itself from the chunk statistics (no barrier before the sums).
 constexpr uint32_t kMergeWaves = 4;
-template <int HD>
+template <int HD, bool FIX>
 __global__ void __launch_bounds__(64 * kMergeWaves) k_attn_merge(AttnArgs a0) {
   const AttnArgs a = attn_query(a0);
   constexpr uint32_t KC = (kAttnMaxChunks + 63) / 64, B = 32;
@@ -568,7 +576,7 @@ __global__ void __launch_bounds__(64 * kMergeWaves) k_attn_merge(AttnArgs a0) {
   __shared__ float s_o[kMergeWaves][64];
   const uint32_t h = blockIdx.x, lane = threadIdx.x & 63, d = blockIdx.y * 64 + lane;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t pos = a.state->pos + blockIdx.z, nch = a.n_chunks;
+  const uint32_t pos = attn_pos<FIX>(a) + blockIdx.z, nch = a.n_chunks;
   const float* ml = a.part_ml + size_t(h) * nch * 2;
   const float* acc = a.part_acc + size_t(h) * nch * HD + d;
   float mv[KC], lv[KC], av[B];
@@ -631,10 +639,12 @@ __global__ void __launch_bounds__(64 * kMergeWaves) k_attn_merge(AttnArgs a0) {
 
 }  // namespace
 
-void launch_attention_partial(const AttnArgs& a, hipStream_t st) {
+namespace {
+template <bool FIX>
+void launch_partial(const AttnArgs& a, hipStream_t st) {
   const uint32_t nq = a.nq > 1 ? a.nq : 1;
   const dim3 grid(a.n_chunks, a.KV, nq);
-  // fp16 cache, a block of more than 8 queries (the prefill): kAttnQz queries per workgroup over
+  // fp16 cache, a block of more than 8 queries: kAttnQz queries per workgroup over
   // one load of its K / V rows (the verify's few queries run in parallel workgroups)
   const bool mq = a.kv_f16 && nq > kSmallBlock;
   const dim3 grid_mq(a.n_chunks, a.KV, (nq + kAttnQz - 1) / kAttnQz);
@@ -642,24 +652,29 @@ void launch_attention_partial(const AttnArgs& a, hipStream_t st) {
   // (the chunk size a.chunk = attn_chunk(hd, KV) picks the instance: CH = waves x positions)
   if (a.hd == 128 && gq == 8 && a.chunk == 128) {  // fp16: 4 waves x 2 tiles; f32: 8 waves x 16 positions
     if (mq) launch_kernel(&k_attn_mq<kAttnMqQz>, dim3(a.n_chunks, a.KV, (nq + kAttnMqQz - 1) / kAttnMqQz), dim3(256), st, a);
-    else if (a.kv_f16) launch_kernel(&k_attn_mfma<128, 8, 4, 2, 1>, grid, dim3(256), st, a);
-    else launch_kernel(&k_attn_chunk<128, 8, float, 4, 8>, grid, dim3(512), st, a);
+    else if (a.kv_f16) launch_kernel(&k_attn_mfma<128, 8, 4, 2, 1, FIX>, grid, dim3(256), st, a);
+    else launch_kernel(&k_attn_chunk<128, 8, float, 4, 8, FIX>, grid, dim3(512), st, a);
   } else if (a.hd == 128 && gq == 8) {  // 64: fp16 4 waves x 1 tile; f32 4 waves x 16 positions, 4 lanes per K row
-    if (mq) launch_kernel(&k_attn_mfma<128, 8, 4, 1, kAttnQz>, grid_mq, dim3(256), st, a);
-    else if (a.kv_f16) launch_kernel(&k_attn_mfma<128, 8, 4, 1, 1>, grid, dim3(256), st, a);
-    else launch_kernel(&k_attn_chunk<128, 8, float, 4, 4>, grid, dim3(256), st, a);
+    if (mq) launch_kernel(&k_attn_mfma<128, 8, 4, 1, kAttnQz, false>, grid_mq, dim3(256), st, a);
+    else if (a.kv_f16) launch_kernel(&k_attn_mfma<128, 8, 4, 1, 1, FIX>, grid, dim3(256), st, a);
+    else launch_kernel(&k_attn_chunk<128, 8, float, 4, 4, FIX>, grid, dim3(256), st, a);
   } else if (a.hd == 256 && gq == 4) {  // fp16: 2 waves x 1 tile; f32: 2 waves x 16 positions
-    if (mq) launch_kernel(&k_attn_mfma<256, 4, 2, 1, kAttnQz>, grid_mq, dim3(128), st, a);
-    else if (a.kv_f16) launch_kernel(&k_attn_mfma<256, 4, 2, 1, 1>, grid, dim3(128), st, a);
-    else launch_kernel(&k_attn_chunk<256, 4, float, 4, 2>, grid, dim3(128), st, a);
+    if (mq) launch_kernel(&k_attn_mfma<256, 4, 2, 1, kAttnQz, false>, grid_mq, dim3(128), st, a);
+    else if (a.kv_f16) launch_kernel(&k_attn_mfma<256, 4, 2, 1, 1, FIX>, grid, dim3(128), st, a);
+    else launch_kernel(&k_attn_chunk<256, 4, float, 4, 2, FIX>, grid, dim3(128), st, a);
   }
 }
 
-void launch_attention_combine(const AttnArgs& a, hipStream_t st) {
+template <bool FIX>
+void launch_combine(const AttnArgs& a, hipStream_t st) {
   const uint32_t nq = a.nq > 1 ? a.nq : 1;
-  if (a.hd == 128) launch_kernel(&k_attn_merge<128>, dim3(a.H, 2, nq), dim3(64 * kMergeWaves), st, a);
-  else launch_kernel(&k_attn_merge<256>, dim3(a.H, 4, nq), dim3(64 * kMergeWaves), st, a);
+  if (a.hd == 128) launch_kernel(&k_attn_merge<128, FIX>, dim3(a.H, 2, nq), dim3(64 * kMergeWaves), st, a);
+  else launch_kernel(&k_attn_merge<256, FIX>, dim3(a.H, 4, nq), dim3(64 * kMergeWaves), st, a);
 }
+}  // namespace
+
+void launch_attention_partial(const AttnArgs& a, hipStream_t st) { launch_partial<false>(a, st); }
+void launch_attention_combine(const AttnArgs& a, hipStream_t st) { launch_combine<false>(a, st); }
 
 bool attention_supported(uint32_t H, uint32_t KV, uint32_t hd) {
   return KV > 0 && H % KV == 0 && ((hd == 128 && H / KV == 8) || (hd == 256 && H / KV == 4));
@@ -672,8 +687,8 @@ void launch_attention(const AttnArgs& a, hipStream_t st) {
 
 // ---- the decode attention on caller buffers with no allocation ------------------------------
 // The chunk kernels' partials (max and sum per chunk and query head, and the weighted V rows)
-// and the position they read live in `scratch`, a file-scope device array: each GPU holds its
-// own copy.  Host code never passes the array's name to a kernel (on the host it is a stand-in,
+// live in `scratch`, a file-scope device array: each GPU holds its own copy.  The position is a
+// kernel argument (a launch of its own to store it cost 1.9 of 12.3 us a call at 3B shapes, position 701).  Host code never passes the array's name to a kernel (on the host it is a stand-in,
 // not a device address): the device address of each GPU's copy is looked up once, with that
 // device current, and kept in g_scratch_ptr.
 namespace {
@@ -684,12 +699,6 @@ constexpr int kMaxDevices = 64;
 void* g_scratch_ptr[kMaxDevices] = {};
 std::once_flag g_scratch_once[kMaxDevices];
 hipError_t g_scratch_err[kMaxDevices] = {};
-
-__global__ void k_set_position(StepState* st, uint32_t pos) {
-  StepState s{};
-  s.pos = pos;
-  *st = s;
-}
 
 }  // namespace
 
@@ -716,16 +725,14 @@ extern "C" int chpe_attention_noalloc(uint32_t head_dim, uint32_t heads, uint32_
   if (max_seq == 0 || max_seq % 16 != 0 || pos >= max_seq) return -1;
   const uint32_t chunk = attn_chunk(head_dim, kv_heads), n_chunks = (pos + chunk) / chunk;
   const size_t ml = size_t(heads) * n_chunks * 2 * 4, acc = size_t(heads) * n_chunks * head_dim * 4;
-  // the position, then the two partial arrays, each at a 256-byte boundary
+  // (256 bytes, then) the two partial arrays, each at a 256-byte boundary
   const size_t off_ml = 256, off_acc = off_ml + (ml + 255) / 256 * 256;
   if (n_chunks > kAttnMaxChunks || off_acc + acc > kAttnScratchBytes) return -2;
   uint8_t* base = static_cast<uint8_t*>(scratch_on_current_device());
   if (!base) return -3;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  StepState* state = reinterpret_cast<StepState*>(base);
-  hipLaunchKernelGGL(k_set_position, dim3(1), dim3(1), 0, st, state, pos);
   AttnArgs a{};
-  a.state = state;
+  a.pos = pos;
   a.q = q;
   a.k_cache = k_cache;
   a.v_cache = v_cache;
@@ -740,6 +747,7 @@ extern "C" int chpe_attention_noalloc(uint32_t head_dim, uint32_t heads, uint32_
   a.chunk = chunk;
   a.kv_f16 = kv_f16 ? 1 : 0;
   a.scale = 1.0f / std::sqrt(float(head_dim));
-  launch_attention(a, st);
+  launch_partial<true>(a, st);
+  launch_combine<true>(a, st);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }

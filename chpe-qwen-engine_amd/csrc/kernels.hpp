@@ -183,7 +183,8 @@ struct EmbedArgs {
 };
 
 struct AttnArgs {
-  const StepState* state;
+  const StepState* state;   // the position (or null: `pos`, the calls with no state)
+  uint32_t pos;
   const float* q;           // [H*hd] rotated queries (the QkvRope GEMV's output)
   const void* k_cache;      // this layer: [KV][max_seq][hd], f16 or f32, rows 0..pos written
   const void* v_cache;      // f32: as k_cache; f16: [KV][max_seq/4][hd][4] (4-position blocks)
