@@ -294,12 +294,16 @@ bool Engine::init(const uint8_t* b, size_t len, const EngineConfig& cfg, std::st
       *err = "block step: " + why;
       return false;
     }
+  }
+  build_xm_layouts();  // the gate/up and LM head codes in the matrix-core kernel's load order
+  {  // the panels (after everything the decode step reads; CHPE_BLOCK=0: off)
+    const char* bk = std::getenv("CHPE_BLOCK");
+    std::string why;
     if (!(bk && bk[0] == '0') && !plan_panel(&why) && !why.empty()) {
       *err = "panels: " + why;
       return false;
     }
   }
-  build_xm_layouts();  // the gate/up and LM head codes in the matrix-core kernel's load order
   HIP_TRY(hipDeviceSynchronize());
 
   // ---- capture the step (CHPE_GRAPH=0 launches the same kernels directly on the stream,
@@ -939,7 +943,20 @@ int Engine::sync() { return hipStreamSynchronize(stream_) == hipSuccess ? 0 : -3
 int Engine::forward_tokens(const uint32_t* toks, size_t n, ForwardResult* out) {
   if (n == 0 || !toks) return -1;
   if (n > cfg_.max_seq_len) return -2;
-  if (panel_ok_ && n >= 2) return prompt_forward(toks, n, out);  // (one position: the decode step's kernels are faster)
+  // A few positions: decode steps (the 3B model's three take 3.2 ms, a block step 3.6, a panel 4.6; the 9B
+  // hybrid's 5.3, 3.8, 5.6).  Up to kSmallBlock: the block step.  More: panels (24 positions of the hybrid:
+  // 42 ms as steps, 6.1 as a block step, 5.6 as a panel).  fp16 raw archives, with no block step, take
+  // panels from three positions on (6.3 ms as steps, 4.9).
+  if (block_ok_ && n > 3 && n <= kSmallBlock) {
+    uint32_t am[kSmallBlock];
+    if (const int rc = block_forward(toks, n, 0, am, out)) return rc;
+    if (set_state(StepState{out->argmax_token, uint32_t(n), 0, 0})) return -3;
+    if (hipMemcpyAsync(embed_fused_ ? d_hidden_out_ : d_hidden_, d_bx_ + (n - 1) * arch_.hidden_dim, arch_.hidden_dim * 4,
+                       hipMemcpyDeviceToDevice, stream_) != hipSuccess)
+      return -3;
+    return sync();
+  }
+  if (panel_ok_ && n > (block_ok_ ? 3u : 2u)) return prompt_forward(toks, n, out);
   if (hipMemcpyAsync(d_prompt_, toks, n * 4, hipMemcpyHostToDevice, stream_) != hipSuccess) return -3;
   if (set_state(StepState{toks[0], 0, uint32_t(n), 0})) return -3;
   if (launch_steps(n - 1)) return -3;
