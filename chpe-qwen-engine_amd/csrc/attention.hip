@@ -422,7 +422,7 @@ __global__ void __launch_bounds__(NW * 64) k_attn_mfma(AttnArgs a) {
   }  // (query z)
 }
 
-// A block step of more than 8 queries (the prefill), fp16 cache, head dim 128, 8 query heads per
+// A block step of more than 8 queries, fp16 cache, head dim 128, 8 query heads per
 // kv head: workgroup (chunk c of 128 positions, kv head, QZ queries).  The chunk's K rows and V
 // blocks are staged in LDS once; wave w then takes queries w, w + 4, ... of the QZ, each over all
 // 128 positions with k_attn_mfma's arithmetic and operand layouts (the operands read from LDS:

@@ -1,6 +1,6 @@
 // block.hip -- the block step's GEMV: m <= kMaxBlock tokens at consecutive positions through
 // flat 4- or 2-bit tiles (gemvCellFlat, chpe_engine.zig:584-729), every weight read once for all
-// of them.  Used by the batch-M verify and by the chunked prefill; each token's arithmetic is the
+// of them.  Used by the batch-M verify and by prompts of up to 32 positions; each token's arithmetic is the
 // batch-1 step's (forwardDecode :1663-1803).
 //
 // 1. k_block_limbs: per token the GEMV input (RMS-normalised, (x * inv) * gamma, rmsNorm
@@ -319,7 +319,7 @@ __global__ void __launch_bounds__(kWave * NW) k_gemv_mt(BlockGemvArgs a) {
   }
 }
 
-// Blocks of 9 .. kMaxBlock tokens (the prefill): output-stationary.  A workgroup of kGmWaves
+// Blocks of 9 .. kMaxBlock tokens: output-stationary.  A workgroup of kGmWaves
 // waves owns a row block of kGmWaves * U units (wave w: units U w .. U w + U - 1 of the block)
 // and one range of column chunks (GC groups each: 128 code bytes of a row for 4-bit GC = 2).
 // Per chunk:

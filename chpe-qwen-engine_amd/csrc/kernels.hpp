@@ -281,7 +281,7 @@ uint32_t launch_gemv_flat_poly(const GemvArgs& a, const uint32_t* n_tiles, float
                                float* part, hipStream_t stream);
 
 // ---- the block step: m <= kMaxBlock tokens at consecutive positions through flat 4- or 2-bit tiles,
-// every weight read once for all m tokens (batch-M verify, chunked prefill) ----------------------
+// every weight read once for all m tokens (batch-M verify, short prompts) ----------------------
 constexpr uint32_t kMaxBlock = 32;
 constexpr uint32_t kSmallBlock = 8;     // blocks up to this size: k_gemv_mt, token stride 8
 constexpr uint32_t kBlockRange = 2048;  // input columns per workgroup of the block GEMV (<= 8 tokens)
