@@ -184,7 +184,6 @@ struct EmbedArgs {
 
 struct AttnArgs {
   const StepState* state;   // the position (or null: `pos`, the calls with no state)
-  uint32_t pos;
   const float* q;           // [H*hd] rotated queries (the QkvRope GEMV's output)
   const void* k_cache;      // this layer: [KV][max_seq][hd], f16 or f32, rows 0..pos written
   const void* v_cache;      // f32: as k_cache; f16: [KV][max_seq/4][hd][4] (4-position blocks)
@@ -197,6 +196,7 @@ struct AttnArgs {
   float scale;              // 1/sqrt(hd)
   uint32_t nq;              // queries of a block step at positions pos .. pos + nq - 1 (rows of q,
                             // out and the partials follow each other); 0 or 1: one query
+  uint32_t pos;             // the position where state is null (here: the pointers stay one 32-byte scalar load)
   const float* gate;        // or null: the merge writes out * sigmoid(g), g the hybrid's output gate
                             //   (query z, head h: gate[z][h][hd + d] of rows [H][2 hd] per query)
 };

@@ -98,3 +98,14 @@ def test_flat_gemv_hook_rejects_bad_arguments_before_the_device():
     for kw in bad:
         with pytest.raises(ca.EngineError):
             ca.gpu_gemv_flat(**kw)
+
+
+def test_step_attention_is_a_code_object_of_its_own():
+    """The engine's attention kernels (the position from the device state) and chpe_attention_noalloc's
+    (the position an argument, the `true` instances) are built from two files: in one code object they
+    slowed every launch of the decode step (attention_call.hip)."""
+    objs = {n: ca.PKG_DIR / "_build" / n for n in ("attention.o", "attention_call.o")}
+    if not all(p.exists() for p in objs.values()):
+        pytest.skip("no build folder")
+    names = {n: set(re.findall(rb"k_attn_(?:mfma|chunk|merge)I\w*?Lb([01])EE", p.read_bytes())) for n, p in objs.items()}
+    assert names == {"attention.o": {b"0"}, "attention_call.o": {b"1"}}
