@@ -715,8 +715,9 @@ __global__ void __launch_bounds__(256) k_panel_epi(PanelEpiArgs a) {
 // neither scores nor weights leave the registers.  fp16 cache: query and weights as hi + lo (each
 // row's query scaled so that its largest value is near 2^14, weights scaled by 2^14), two products
 // each; f32 cache: f32 products.  In the last steps, where some of the wave's tokens see a
-// position and others do not, each token runs alone with the positions past it taken out of V
-// (0 times a non-finite row is not 0).
+// position and others do not, each token runs alone with the positions past it taken out of V, and only
+// its own rows keep the sums (0 times a non-finite row is not 0, neither for the token itself nor for the
+// ones before it, which do not see that row).
 constexpr float kPUp = 16384.0f;
 
 struct SoftRow {
@@ -895,9 +896,7 @@ __global__ void __launch_bounds__(256) k_panel_attn_h(PanelAttnArgs a) {
       }
     } else {
       for (uint32_t u = 0; u < uint32_t(TT); ++u) {
-        const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
         const bool mine = n / G == u;
-        const half8_t Pu = mine ? Ph : zero, Pv = mine ? Pl : zero;
         const uint32_t last = first + u < pmax ? first + u : pmax;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
@@ -908,8 +907,10 @@ __global__ void __launch_bounds__(256) k_panel_attn_h(PanelAttnArgs a) {
             x[k] = (p <= last ? x[k] & 0xFFFFu : 0u) | (p + 1 <= last ? x[k] & 0xFFFF0000u : 0u);
           }
           const half8_t V = as_half8(make_uint4(x[0], x[1], x[2], x[3]));
-          O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(V, Pv, O[dt], 0, 0, 0);
-          O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(V, Pu, O[dt], 0, 0, 0);
+          f32x4_t R = __builtin_amdgcn_mfma_f32_16x16x32_f16(V, Pl, O[dt], 0, 0, 0);
+          R = __builtin_amdgcn_mfma_f32_16x16x32_f16(V, Ph, R, 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) O[dt][j] = mine ? R[j] : O[dt][j];
         }
       }
     }
@@ -1004,12 +1005,13 @@ __global__ void __launch_bounds__(256) k_panel_attn_f(PanelAttnArgs a) {
         const bool mine = n / G == u;
         const uint32_t last = first + u < pmax ? first + u : pmax;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const bool in = p0 + 4 * q + uint32_t(j) <= last;
-          const float eu = mine ? e[j] : 0.0f;
+        for (int dt = 0; dt < DT; ++dt) {
+          f32x4_t R = O[dt];
 #pragma unroll
-          for (int dt = 0; dt < DT; ++dt)
-            O[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? vv[j][dt] : 0.0f, eu, O[dt], 0, 0, 0);
+          for (int j = 0; j < 4; ++j)
+            R = __builtin_amdgcn_mfma_f32_16x16x4f32(p0 + 4 * q + uint32_t(j) <= last ? vv[j][dt] : 0.0f, e[j], R, 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) O[dt][j] = mine ? R[j] : O[dt][j];
         }
       }
     }

@@ -11,6 +11,8 @@ bars four times that.  An argmax may differ only where the two best logits are c
 than the bar.  (The 72B archives' panels: test_gpu_models.py, a prompt of 11 against the block step
 and the oracle.)"""
 import os
+import shutil
+import tempfile
 
 import numpy as np
 import pytest
@@ -76,8 +78,6 @@ def test_panel_break(w4_archive, monkeypatch):
     """forwardDecode's non-finite break (StepState::broken) in a panel: an infinite outlier weight
     in layer 1's down projection stops every token after that layer; the final norm and the LM head
     see that hidden state, as in the decode steps."""
-    import tempfile
-
     import oracle as orc
     from test_gpu_nonfinite import inf_outlier_edit
     li = orc.layer_info(1, 1)
@@ -100,6 +100,47 @@ def test_panel_break(w4_archive, monkeypatch):
             assert np.array_equal(np.isfinite(hid), fin) and rel(hid[fin], hid0[fin]) <= 4e-5
             assert np.array_equal(np.isnan(got), np.isnan(want)) and am == am0
             assert last["hidden_norm"] == last0["hidden_norm"] == np.inf
+        finally:
+            e.close()
+            steps.close()
+    finally:
+        os.unlink(path)
+
+
+@pytest.mark.timeout(300)
+@pytest.mark.parametrize("kind,arch,vocab,kv16,at,bar", [
+    (ca.PACK_3B_W4, 0, 151936, False, 21, 4e-5), (ca.PACK_3B_W4, 0, 151936, True, 21, 8e-4),
+    (ca.PACK_9B_W4, 1, 248320, False, 23, 8e-5), (ca.PACK_9B_W4, 1, 248320, True, 23, 8e-4)])
+def test_panel_nonfinite_row(kind, arch, vocab, kv16, at, bar, monkeypatch):
+    """A token whose embedding row is not finite writes NaN keys and values into layer 0's cache; the
+    attention of the tokens before it in the same tile of 16 rows (2 tokens of 8 heads, 4 of 4) must not
+    meet them: a decode step that goes back to its position reads the rows before it, finite and as the
+    decode steps left them.  (`at`: the last token of a tile.)"""
+    bad, src = 1234, archive_path(kind)
+    fd, path = tempfile.mkstemp(suffix=".chpe", prefix="qwen2.5-3b-mod-" if arch == 0 else "qwen3.5-9b-mod-",
+                                dir=os.path.dirname(str(src)))
+    os.close(fd)
+    shutil.copyfile(src, path)
+    cell = 4096 + bad // 16 * 17408 + 64 + 16384
+    with open(path, "r+b") as f:  # 3B: the row's last outlier value; 9B: the tile's offset (16 tokens' rows)
+        f.seek(cell + 560 + 16 * (bad % 16) + 14 if arch == 0 else cell + 36)
+        f.write(np.float16(np.inf).tobytes() if arch == 0 else np.float32(np.inf).tobytes())
+    try:
+        e, steps = engines(path, arch, 64, kv16, monkeypatch)
+        try:
+            toks = np.random.default_rng(11).integers(2000, vocab, 40).astype(np.uint32)
+            toks[at] = bad
+            hid, nxt = [], []
+            for x in (steps, e):
+                x.forward_tokens(toks)
+                hid.append(x.hidden())
+                nxt.append(x.decode_step(2001, at)[1])
+            fin = np.isfinite(nxt[0])
+            assert not np.isfinite(hid[0]).any() and not np.isfinite(hid[1]).any()
+            assert fin.sum() >= vocab - 16 and np.array_equal(np.isfinite(nxt[1]), fin)
+            d = rel(nxt[1][fin], nxt[0][fin])
+            print(f"arch {arch} kv16 {kv16}: the step at {at}: {d:.2e}", flush=True)
+            assert d <= bar
         finally:
             e.close()
             steps.close()
