@@ -472,10 +472,14 @@ __global__ void __launch_bounds__(256, 1) k_panel_gemm(PanelGemmArgs a) {
 }
 
 // fp16 weights: v_mfma_f32_16x16x32_f16, D lane (n, q) = row n, tokens 4 q .. + 3; the k slots of step
-// d hold columns 32 q + 8 d .. + 7.  The products are exact; the small parts' sums go first (no rounding
-// near the group's size), each step of the high parts has an f32 sum of its own, and those are added up
-// in 64 bits (measured on random weights, 128 columns: 0.74 x 2^-24 of the sum, against 1.29 in one
-// chain).  U = 2 units per wave: 64 bytes of codes per lane, unit and group.
+// d hold columns 32 q + 8 d .. + 7.  The products are exact; the small parts have a sum of their own, each
+// step of 16 columns of the high parts has one, and those are added up in 64 bits (measured on random
+// weights, 128 columns: 0.74 x 2^-24 of the sum, against 1.29 in one chain).  U = 2 units per wave:
+// 64 bytes of codes per lane, unit and group.
+// The small parts' sum is not the starting value of the first 16 columns' product: that is another opcode, and
+// the compiler puts no wait between two products that hand on exactly the same registers.  Where its
+// schedule brought the 16x16x16 product within 32 cycles of the 16x16x32 one it starts from, the sum was
+// taken too early (the last small part missing) and the logits were 2e-5 to 2e-4 off.
 struct PanelHalves {
   uint4 v[2][4];
 };
@@ -530,12 +534,18 @@ __global__ void __launch_bounds__(256, 2) k_panel_gemm_h(PanelGemmArgs a) {
           const half8_t B = as_half8(c.v[u][d]);
           const half4_t B0 = __builtin_shufflevector(B, B, 0, 1, 2, 3), B1 = __builtin_shufflevector(B, B, 4, 5, 6, 7);
           const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-          const f32x4_t E0 = __builtin_amdgcn_mfma_f32_16x16x16f16(A0, B0, d == 0 ? D[u][t] : z, 0, 0, 0);
+          const f32x4_t E0 = __builtin_amdgcn_mfma_f32_16x16x16f16(A0, B0, z, 0, 0, 0);
           const f32x4_t E1 = __builtin_amdgcn_mfma_f32_16x16x16f16(A1, B1, z, 0, 0, 0);
 #pragma unroll
           for (int j = 0; j < 4; ++j) acc[u][t][j] += double(E0[j]) + double(E1[j]);
         }
       }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[u][t][j] += double(D[u][t][j]);
   };
   panel_loop_near<PanelHalves>(p, s_x0, s_x1, issue, fetch, compute);
   f32x4_t sum[U][TT];
