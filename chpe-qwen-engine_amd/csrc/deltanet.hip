@@ -477,20 +477,11 @@ __global__ void __launch_bounds__(256) k_dn_gnorm_block(DnBlockArgs a) {
     o[k] = *reinterpret_cast<const float2*>(out + k * D);
     g[k] = *reinterpret_cast<const float2*>(z + k * D);
   }
-  uint32_t mx = 0;
 #pragma unroll
   for (uint32_t k = 0; k < 2; ++k) {
     const float tot = wave_sum(o[k].x * o[k].x + o[k].y * o[k].y);
     const float rr = 1.0f / sqrtf(tot / float(D) + a.eps);
-    const float2 y = make_float2(w.x * (o[k].x * rr) * silu_f(g[k].x), w.y * (o[k].y * rr) * silu_f(g[k].y));
-    *reinterpret_cast<float2*>(out + k * D) = y;
-    const uint32_t bx = __float_as_uint(y.x) & 0x7fffffffu, by = __float_as_uint(y.y) & 0x7fffffffu;
-    mx = mx > bx ? mx : bx;
-    mx = mx > by ? mx : by;
-  }
-  if (a.tokmax) {  // (uniform)
-    mx = lanes_umax<64>(mx);
-    if (lane == 0) atomicMax(&a.tokmax[(blockIdx.x % kPanelMaxSlots) * kMaxPanel + tk], mx);
+    *reinterpret_cast<float2*>(out + k * D) = make_float2(w.x * (o[k].x * rr) * silu_f(g[k].x), w.y * (o[k].y * rr) * silu_f(g[k].y));
   }
 }
 

@@ -1478,17 +1478,14 @@ bool Engine::plan_panel(std::string* err) {
   d_pq_ = fa(M * qd);
   d_pattn_ = fa(M * qd);
   d_pmlp_ = fa(M * I);
-  d_pxs_ = static_cast<uint4*>(dev_alloc(kPanelRows * Cmax * (block_ok_ ? 4 : 6)));  // (limbs; three fp16 parts)
+  // (limbs or three fp16 parts; at most 16 token tiles of kPanelScales scales a group)
+  d_pxs_ = static_cast<uint4*>(dev_alloc(kPanelRows * Cmax * (block_ok_ ? 4 : 6) + 16 * (Cmax / 128) * kPanelScales * 4));
   d_pxt_ = fa(kPanelRows * Cmax);
   d_ppart_ = fa(ppart_floats_);
-  d_pdown_ = fa(M);
   d_pss_ = fa((D + 15) / 16 * M);
-  d_pmx_ = static_cast<uint32_t*>(dev_alloc((D + 15) / 16 * M * 4));
-  d_pmax_ = static_cast<uint32_t*>(dev_alloc(2 * arch_.num_layers * kPanelMaxSlots * M * 4));
   d_pbrk_ = static_cast<uint32_t*>(dev_alloc(M * 4));
   d_pstate_ = static_cast<StepState*>(dev_alloc(sizeof(StepState)));
-  bool ok = d_px_ && d_pq_ && d_pattn_ && d_pmlp_ && d_pxs_ && d_pxt_ && d_ppart_ && d_pdown_ && d_pss_ && d_pmx_ && d_pmax_ &&
-            d_pbrk_ && d_pstate_;
+  bool ok = d_px_ && d_pq_ && d_pattn_ && d_pmlp_ && d_pxs_ && d_pxt_ && d_ppart_ && d_pss_ && d_pbrk_ && d_pstate_;
   if (cfg_.hybrid) {
     d_phx0_ = fa(M * 8192);
     d_phx1_ = fa(M * 4096);
@@ -1506,9 +1503,8 @@ bool Engine::plan_panel(std::string* err) {
 }
 
 uint32_t Engine::enqueue_panel_gemm(const ProjPlan* const* parts, float* const* outs, int n, GemvMode mode,
-                                    const float* x, uint32_t C, const float* gamma, uint32_t n_ss, uint32_t* max_rows,
-                                    const float* gamma_next, uint32_t m, uint32_t pos, size_t layer,
-                                    hipStream_t st, const uint32_t* roles_in, uint32_t pair_dim) {
+                                    const float* x, uint32_t C, const float* gamma, uint32_t n_ss, uint32_t m, uint32_t pos,
+                                    size_t layer, hipStream_t st, const uint32_t* roles_in, uint32_t pair_dim) {
   const uint32_t ng = C / 128;
   const WeightKind kind = parts[0]->kind;
   const uint32_t bits = kind == WeightKind::Raw16 ? 16u : kind == WeightKind::FlatW2 ? 2u : 4u;
@@ -1546,11 +1542,8 @@ uint32_t Engine::enqueue_panel_gemm(const ProjPlan* const* parts, float* const* 
   s.eps = arch_.rms_eps;
   s.ssp = d_pss_;
   s.n_ssp = n_ss;
-  s.tokmax = gamma ? d_pmx_ : max_rows;
-  s.n_max = gamma ? n_ss : kPanelMaxSlots;
   s.xs = d_pxs_;
   s.xt = corr ? d_pxt_ : nullptr;
-  s.down = d_pdown_;
   s.C = C;
   s.m = m;
   s.n_tok = n_tok;
@@ -1577,7 +1570,6 @@ uint32_t Engine::enqueue_panel_gemm(const ProjPlan* const* parts, float* const* 
   e.rows_all = rows_all;
   e.partial = d_ppart_;
   e.xt = d_pxt_;
-  e.down = d_pdown_;
   e.pos = pos;
   e.head_dim = pair_dim ? pair_dim : rope.head_dim;
   e.max_seq = rope.max_seq;
@@ -1588,9 +1580,6 @@ uint32_t Engine::enqueue_panel_gemm(const ProjPlan* const* parts, float* const* 
   e.k_cache = rope.k_cache;
   e.v_cache = rope.v_cache;
   e.ssp_out = d_pss_;
-  e.mx_out = d_pmx_;
-  e.gamma_next = gamma_next;
-  e.tokmax_out = max_rows;
   e.brk = d_pbrk_;
   launch_panel_epi(e, mode, st);
   const uint32_t et = panel_epi_tile(e.total, m);
@@ -1600,22 +1589,18 @@ uint32_t Engine::enqueue_panel_gemm(const ProjPlan* const* parts, float* const* 
 void Engine::enqueue_panel(uint32_t token, uint32_t pos, uint32_t m, hipStream_t st) {
   const uint32_t D = uint32_t(arch_.hidden_dim), I = uint32_t(arch_.intermediate_dim);
   const uint32_t H = uint32_t(arch_.num_attn_heads), KV = uint32_t(arch_.num_kv_heads), hd = uint32_t(arch_.head_dim);
-  launch_panel_begin(PanelBeginArgs{d_pstate_, token, pos, d_pmax_, uint32_t(2 * arch_.num_layers) * kPanelMaxSlots * kMaxPanel}, st);
+  if (cfg_.hybrid) launch_panel_begin(d_pstate_, token, pos, st);  // (launch_hyb_qk's first position)
   launch_block_embed(embed_args(), d_prompt_ + pos, m, d_px_, d_pss_, d_pbrk_, st);
-  launch_panel_rowmax(d_px_, layers_[0].gamma_in, D, m, d_pmx_, st);
-  uint32_t n_ss = 1;  // partial sums and maxima of the hidden rows
+  uint32_t n_ss = 1;  // partial sums of the hidden rows
   float* hid[1] = {d_px_};
   for (size_t l = 0; l < arch_.num_layers; ++l) {
     const LayerPlan& L = layers_[l];
-    uint32_t* max_attn = d_pmax_ + 2 * l * kPanelMaxSlots * kMaxPanel;
-    uint32_t* max_mlp = max_attn + kPanelMaxSlots * kMaxPanel;
     const RopeArgs kv = rope_args(l);
     PanelAttnArgs at{};
     at.q = d_pq_;
     at.k_cache = kv.k_cache;
     at.v_cache = kv.v_cache;
     at.out = d_pattn_;
-    at.tokmax_out = max_attn;
     at.H = H;
     at.KV = KV;
     at.hd = hd;
@@ -1627,17 +1612,17 @@ void Engine::enqueue_panel(uint32_t token, uint32_t pos, uint32_t m, hipStream_t
     if (!cfg_.hybrid) {
       const ProjPlan* qkv[3] = {&L.q, &L.k, &L.v};
       float* qo[3] = {d_pq_, nullptr, nullptr};
-      enqueue_panel_gemm(qkv, qo, 3, GemvMode::QkvRope, d_px_, D, L.gamma_in, n_ss, nullptr, nullptr, m, pos, l, st);
+      enqueue_panel_gemm(qkv, qo, 3, GemvMode::QkvRope, d_px_, D, L.gamma_in, n_ss, m, pos, l, st);
       launch_panel_attention(at, st);
       const ProjPlan* o[1] = {&L.o};
-      n_ss = enqueue_panel_gemm(o, hid, 1, GemvMode::Accum, d_pattn_, D, nullptr, 0, max_attn, L.gamma_post, m, pos, l, st);
+      n_ss = enqueue_panel_gemm(o, hid, 1, GemvMode::Accum, d_pattn_, D, nullptr, 0, m, pos, l, st);
     } else {
       const HybLayer& Hy = hyb_[l];
       const uint32_t store[3] = {kRoleStore, kRoleStore, kRoleStore};
       const bool ab = !Hy.full && Hy.has_ab;
       const ProjPlan* in[3] = {&Hy.in0, &Hy.in1, ab ? &Hy.ab : &Hy.in2};
       float* outs[3] = {d_phx0_, d_phx1_, d_phx2_};
-      enqueue_panel_gemm(in, outs, 3, GemvMode::QkvRope, d_px_, D, L.gamma_in, n_ss, nullptr, nullptr, m, pos, l, st,
+      enqueue_panel_gemm(in, outs, 3, GemvMode::QkvRope, d_px_, D, L.gamma_in, n_ss, m, pos, l, st,
                          store, 32);
       if (Hy.full) {
         launch_hyb_qk(hyb_qk_args(l, d_pstate_, d_phx0_, d_phx1_, d_phx2_, d_pq_, d_pbrk_, m), st);
@@ -1647,22 +1632,19 @@ void Engine::enqueue_panel(uint32_t token, uint32_t pos, uint32_t m, hipStream_t
         if (!ab) {
           const ProjPlan* inb[1] = {&Hy.in3};
           float* outb[1] = {d_phx3_};
-          enqueue_panel_gemm(inb, outb, 1, GemvMode::QkvRope, d_px_, D, L.gamma_in, n_ss, nullptr, nullptr, m, pos, l, st,
+          enqueue_panel_gemm(inb, outb, 1, GemvMode::QkvRope, d_px_, D, L.gamma_in, n_ss, m, pos, l, st,
                              store, 32);
         }
-        DnBlockArgs dn = dn_block_args(l, d_phx0_, d_phx1_, d_phx2_, d_phx3_, d_phconv_, d_pattn_, d_pbrk_, m);
-        dn.tokmax = max_attn;
-        launch_dn_block(dn, st);
+        launch_dn_block(dn_block_args(l, d_phx0_, d_phx1_, d_phx2_, d_phx3_, d_phconv_, d_pattn_, d_pbrk_, m), st);
       }
       const ProjPlan* o[1] = {&Hy.out};
-      n_ss = enqueue_panel_gemm(o, hid, 1, GemvMode::Accum, d_pattn_, 4096, nullptr, 0, max_attn, L.gamma_post, m, pos, l, st);
+      n_ss = enqueue_panel_gemm(o, hid, 1, GemvMode::Accum, d_pattn_, 4096, nullptr, 0, m, pos, l, st);
     }
     const ProjPlan* gu[2] = {&L.gate, &L.up};
     float* mlp[2] = {d_pmlp_, d_pmlp_};
-    enqueue_panel_gemm(gu, mlp, 2, GemvMode::SwiGlu, d_px_, D, L.gamma_post, n_ss, max_mlp, nullptr, m, pos, l, st);
+    enqueue_panel_gemm(gu, mlp, 2, GemvMode::SwiGlu, d_px_, D, L.gamma_post, n_ss, m, pos, l, st);
     const ProjPlan* dn[1] = {&L.down};
-    const float* gamma_next = l + 1 < arch_.num_layers ? layers_[l + 1].gamma_in : d_gamma_final_;
-    n_ss = enqueue_panel_gemm(dn, hid, 1, GemvMode::Accum, d_pmlp_, I, nullptr, 0, max_mlp, gamma_next, m, pos, l, st);
+    n_ss = enqueue_panel_gemm(dn, hid, 1, GemvMode::Accum, d_pmlp_, I, nullptr, 0, m, pos, l, st);
   }
 }
 

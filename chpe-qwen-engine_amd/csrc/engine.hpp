@@ -244,13 +244,11 @@ class Engine {
   bool plan_panel(std::string* err);
   // m positions pos .. of the prompt (its tokens at d_prompt_ + pos) through every layer
   void enqueue_panel(uint32_t token, uint32_t pos, uint32_t m, hipStream_t st);
-  // a panel's projections of one input.  gamma: the rows' partial sums and maxima are in d_pss_ and
-  // d_pmx_ (n_ss each), where Accum leaves the updated rows' (of |y * gamma_next|); otherwise max_rows
-  // holds their maxima, where SwiGlu leaves its output's.  roles, pair_dim as enqueue_block_gemv
+  // a panel's projections of one input.  gamma: the rows' n_ss partial sums of squares are in d_pss_,
+  // where Accum leaves the updated rows'.  roles, pair_dim as enqueue_block_gemv
   uint32_t enqueue_panel_gemm(const ProjPlan* const* parts, float* const* outs, int n, GemvMode mode, const float* x,
-                              uint32_t C, const float* gamma, uint32_t n_ss, uint32_t* max_rows,
-                              const float* gamma_next, uint32_t m, uint32_t pos, size_t layer, hipStream_t st,
-                              const uint32_t* roles = nullptr, uint32_t pair_dim = 0);
+                              uint32_t C, const float* gamma, uint32_t n_ss, uint32_t m, uint32_t pos, size_t layer,
+                              hipStream_t st, const uint32_t* roles = nullptr, uint32_t pair_dim = 0);
 
  public:
   // run one projection's GEMV on a caller vector (Store mode, bias included): parity hooks
@@ -329,14 +327,14 @@ class Engine {
   // captured block steps, by token count
   hipGraph_t bgraph_[kMaxBlock + 1] = {};
   hipGraphExec_t bgraph_exec_[kMaxBlock + 1] = {};
-  // the panels (plan_panel): activations of kMaxPanel rows, the GEMM's fp16 input images, partial
-  // sums, per-token scales, maxima [2 per layer][kPanelMaxSlots][kMaxPanel] and break flags
+  // the panels (plan_panel): activations of kMaxPanel rows, the GEMM's input images, partial sums and
+  // break flags
   bool panel_ok_ = false;
   float *d_px_ = nullptr, *d_pq_ = nullptr, *d_pattn_ = nullptr, *d_pmlp_ = nullptr, *d_pxt_ = nullptr;
-  float *d_ppart_ = nullptr, *d_pdown_ = nullptr, *d_pss_ = nullptr;
+  float *d_ppart_ = nullptr, *d_pss_ = nullptr;
   float *d_phx0_ = nullptr, *d_phx1_ = nullptr, *d_phx2_ = nullptr, *d_phx3_ = nullptr, *d_phconv_ = nullptr;
   uint4* d_pxs_ = nullptr;
-  uint32_t *d_pmax_ = nullptr, *d_pmx_ = nullptr, *d_pbrk_ = nullptr;
+  uint32_t* d_pbrk_ = nullptr;
   StepState* d_pstate_ = nullptr;
   size_t ppart_floats_ = 0;
   int probe_stage_ = -1;                 // stage bracketed by events in record_step

@@ -408,7 +408,6 @@ struct DnBlockArgs {
   uint32_t n_v_heads, n_k_heads, head_dim, m;
   float eps;
   const uint32_t* brk;      // [m]: token t broke before this layer (its state updates are skipped)
-  uint32_t* tokmax;         // or null: [kPanelMaxSlots][kMaxPanel] maxima of |out|
 };
 void launch_dn_block(const DnBlockArgs& a, hipStream_t stream);
 
@@ -461,27 +460,18 @@ constexpr uint32_t kMaxLogitsBlocks = 8192;
 // ---- panels: up to kMaxPanel tokens of a prompt at consecutive positions (panel.hip) ------------
 constexpr uint32_t kMaxPanel = 512;
 constexpr uint32_t kPanelRows = kMaxPanel + 112;  // rows of the GEMM's buffers: m in whole tiles of up to 112 tokens
-// Attention and the SwiGLU leave the largest |value| of each row as atomic maxima (of the bits) in
-// kPanelMaxSlots rows of [kMaxPanel] (a workgroup uses one of them: in a single row of 32 tokens to a cache line the 688
-// workgroups of a SwiGLU launch queue on one line, 45 us instead of 6)
-constexpr uint32_t kPanelMaxSlots = 16;
-struct PanelBeginArgs {    // the panel's state and cleared maxima
-  StepState* state;
-  uint32_t token, pos;
-  uint32_t* tokmax;        // [n_max]
-  uint32_t n_max;
-};
+// 16-byte pieces of one 128-column group of a token tile as the GEMM's operands: four limbs of a byte or three
+// fp16 parts, then the tokens' scales (kPanelScales floats, at most 112 of them used: one 4-byte load of 256 lanes)
+constexpr uint32_t kPanelScales = 256;
+constexpr uint32_t panel_image(uint32_t tile, uint32_t bits) { return tile * (bits == 16 ? 48 : 32) + kPanelScales / 4; }
 struct PanelSplitArgs {    // a GEMM's input rows as matrix-core operands
   const float* x;          // [m][C]
   const float* gamma;      // RMSNorm gains, or null
   float eps;
   const float* ssp;        // (gamma) [n_ssp][kMaxPanel]: partial sums of x^2 of the rows
   uint32_t n_ssp;
-  const uint32_t* tokmax;  // [n_max][kMaxPanel]: partial maxima, as bits, of |x| (gamma: of |x * gamma|) of the rows
-  uint32_t n_max;
-  uint4* xs;               // [token tile][group]: the GEMM's LDS images (k_panel_split)
+  uint4* xs;               // [token tile][group][panel_image]: the GEMM's LDS images (k_panel_split)
   float* xt;               // [C][n_tok] f32, token-minor, or null
-  float* down;             // [m]: the factor from a row's products to its values
   uint32_t C, m, n_tok, tile;  // n_tok: m rounded up to whole token tiles
   uint32_t* brk;           // [m] break flags, set by the test chk (RopeArgs::brk_check)
   uint32_t chk;
@@ -508,14 +498,10 @@ struct PanelEpiArgs {
   uint32_t m, n_tok, ranges, rows_all, total;  // total: outputs (rows of part 0; RoPE pairs of all parts)
   const float* partial;
   const float* xt;
-  const float* down;
   uint32_t pos, head_dim, max_seq, kv_f16, rope_rows;
   const float *rope_cos, *rope_sin;
   void *k_cache, *v_cache;
-  float* ssp_out;          // Accum: [total / panel_epi_tile][kMaxPanel] partial sums of y^2,
-  uint32_t* mx_out;        //   and maxima of |y * gamma_next|
-  const float* gamma_next; //   (the gains of the norm that reads the rows next)
-  uint32_t* tokmax_out;    // SwiGlu: [kPanelMaxSlots][kMaxPanel] maxima of |y|
+  float* ssp_out;          // Accum: [total / panel_epi_tile][kMaxPanel] partial sums of y^2
   const uint32_t* brk;
 };
 struct PanelAttnArgs {
@@ -523,12 +509,10 @@ struct PanelAttnArgs {
   const void *k_cache, *v_cache;  // as AttnArgs
   float* out;              // [m][H][hd]
   const float* gate;       // or null: as AttnArgs
-  uint32_t* tokmax_out;    // [kPanelMaxSlots][kMaxPanel] maxima of |out|
   uint32_t H, KV, hd, max_seq, kv_f16, pos, m;
   float scale;
 };
-void launch_panel_begin(const PanelBeginArgs& a, hipStream_t stream);
-void launch_panel_rowmax(const float* x, const float* gamma, uint32_t C, uint32_t m, uint32_t* mx_out, hipStream_t stream);
+void launch_panel_begin(StepState* state, uint32_t token, uint32_t pos, hipStream_t stream);  // the panel's first position
 void launch_panel_split(const PanelSplitArgs& a, uint32_t bits, hipStream_t stream);
 void launch_panel_gemm(const PanelGemmArgs& a, uint32_t bits, uint32_t tile, hipStream_t stream);
 void launch_panel_epi(const PanelEpiArgs& a, GemvMode mode, hipStream_t stream);

@@ -1,12 +1,15 @@
 // panel.hip -- a prompt's positions in panels of up to kMaxPanel tokens: every weight is read once
-// per panel and the products run on the matrix cores with both operands in fp16.
+// per panel and the products run on the matrix cores, in 8-bit integers (4- and 2-bit codes) or fp16.
 //
 // Per projection:
 // 1. k_panel_split: the input rows (RMS-normalised, (x * inv) * gamma, rmsNorm :187-191, when gamma
-//    is set) as matrix-core operands.  For 4- and 2-bit codes: X = x * 2^(30 - e), max |x| of the
-//    token < 2^e, in four balanced signed-byte limbs (an error of 2^-31 of the token's largest
-//    value, below what f32 sums over 2048 columns and more resolve).  For fp16 weights: x * 2^(14 - e)
-//    as the sum of three fp16 numbers of 11 bits each, f32's 24 and more.  (Two fp16 numbers carry 23
+//    is set) as matrix-core operands, each 128-column group of a token with a scale of its own, as in
+//    the block step (one scale per token let a channel 2^12 times the others take 12 of their bits).
+//    For 4- and 2-bit codes: X = x * 2^(30 - e), max |x| of the group < 2^e, rounded to nearest, in
+//    four balanced signed-byte limbs: within 2^-30 of the group's largest value (X is exact where
+//    |x| is 2^-6 of it or more), below what f32 sums over 2048 columns and more resolve.  For fp16 weights: x * 2^(14 - e)
+//    as the sum of three fp16 numbers of 11 bits each, f32's 24 bits and more down to 2^-14 of the
+//    group's largest value, within 2^-38 of that below.  (Two fp16 numbers carry 23
 //    bits: half the time the last bit of an f32 is lost, and the logits of the 3B model were 1.25
 //    to 2 times as far from their 64-bit values.)
 // 2. k_panel_gemm / k_panel_gemm_h: workgroup = 256 (128) weight rows x one token tile x a range of
@@ -32,7 +35,7 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {  // (each rounded 
 }
 __device__ __forceinline__ float f16_round(float x) { return float(_Float16(x)); }
 // 2^(b - e) for a largest magnitude below 2^e (given as its bits), kept a normal number; a
-// non-finite magnitude: NaN (every product of the row is then NaN)
+// non-finite magnitude: NaN (every product of the group is then NaN)
 __device__ __forceinline__ float scale_up(uint32_t max_bits, int b) {
   if (max_bits >= 0x7f800000u) return __uint_as_float(0x7fc00000u);
   int e = int(max_bits >> 23) - 126;  // (subnormal maxima: as 2^-126)
@@ -40,29 +43,7 @@ __device__ __forceinline__ float scale_up(uint32_t max_bits, int b) {
   return ldexpf(1.0f, b - e);
 }
 
-__global__ void __launch_bounds__(256) k_panel_begin(PanelBeginArgs a) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i < a.n_max) a.tokmax[i] = 0u;
-  if (i == 0) *a.state = StepState{a.token, a.pos, 0, 0};
-}
-
-// the rows' largest |x * gamma| (the first layer's input: later ones come from k_panel_epi) into
-// mx_out [1][kMaxPanel]; a workgroup per row
-__global__ void __launch_bounds__(256) k_panel_rowmax(const float* x, const float* gamma, uint32_t C, uint32_t* mx_out) {
-  __shared__ uint32_t s_mx[4];
-  uint32_t mx = 0;
-  for (uint32_t c = threadIdx.x; c < C; c += 256) {
-    const uint32_t b = __float_as_uint(x[size_t(blockIdx.x) * C + c] * gamma[c]) & 0x7fffffffu;
-    mx = mx > b ? mx : b;
-  }
-  mx = lanes_umax<64>(mx);
-  if ((threadIdx.x & 63) == 0) s_mx[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const uint32_t p = s_mx[0] > s_mx[1] ? s_mx[0] : s_mx[1], q = s_mx[2] > s_mx[3] ? s_mx[2] : s_mx[3];
-    mx_out[blockIdx.x] = p > q ? p : q;
-  }
-}
+__global__ void k_panel_begin(StepState* state, uint32_t token, uint32_t pos) { *state = StepState{token, pos, 0, 0}; }
 
 // grid (128-column groups, 64-token tiles): 64 tokens x 128 columns.  Thread (token, 8 columns)
 // four times.  The images are what the GEMM copies to LDS linearly, 16-byte pieces placed so that
@@ -70,15 +51,15 @@ __global__ void __launch_bounds__(256) k_panel_rowmax(const float* x, const floa
 //   limbs: [limb][token][8 pieces of 16 columns], piece c of token t at slot c ^ ((t >> 1) & 7), its
 //     columns in the unpacked codes' order (4-bit {0,2,4,6}, {1,3,5,7}, {8,..}, {9,..}; 2-bit
 //     {0,4,8,12}, {1,..}, {2,..}, {3,..}); thread pairs hold the two halves of a piece;
-//   fp16: [part][token][16 pieces of 8 columns], piece c of token t at slot c ^ (t & 15).
+//   fp16: [part][token][16 pieces of 8 columns], piece c of token t at slot c ^ (t & 15);
+//   then kScales floats, the factors from the tokens' products in this group to their values.
 // The f32 values go out token-minor for the outlier corrections, through LDS.  Bound by memory: 4
 // bytes in, 4 + 4 out per element.
 template <bool kNorm, int BITS>
 __global__ void __launch_bounds__(256) k_panel_split(PanelSplitArgs a) {
   __shared__ float s_x[128][65];
   __shared__ double s_red[4][64];
-  __shared__ float s_inv[64], s_up[64];
-  __shared__ uint32_t s_mx[4][64];
+  __shared__ float s_inv[64];
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint32_t g = blockIdx.x, tok0 = blockIdx.y * 64, C = a.C, ng = C >> 7;
   float4 xa[4], xb[4];
@@ -89,47 +70,25 @@ __global__ void __launch_bounds__(256) k_panel_split(PanelSplitArgs a) {
     xa[i] = ld_f4(row);
     xb[i] = ld_f4(row + 4);
   }
-  const uint32_t tl = tok0 + lane < a.m ? tok0 + lane : a.m - 1;
+  [[maybe_unused]] const uint32_t tl = tok0 + lane < a.m ? tok0 + lane : a.m - 1;
   constexpr int kUp = BITS == 16 ? 14 : 30;
-  {  // the producers' partial maxima (and sums of squares), each wave a quarter of them
+  if constexpr (kNorm) {  // the producers' partial sums of squares, each wave a quarter of them
     // (in 64 bits: the norm's factor scales the whole row, its error is not averaged out by the sums)
-    uint32_t mx = 0;
     double ss = 0.0;
 #pragma unroll 8
-    for (uint32_t i = wave; i < a.n_max; i += 4) {
-      const uint32_t v = a.tokmax[size_t(i) * kMaxPanel + tl];
-      mx = mx > v ? mx : v;
-    }
-    if constexpr (kNorm) {
-#pragma unroll 8
-      for (uint32_t i = wave; i < a.n_ssp; i += 4) ss += double(a.ssp[size_t(i) * kMaxPanel + tl]);
-      s_red[wave][lane] = ss;
-    }
-    s_mx[wave][lane] = mx;
-  }
-  __syncthreads();
-  if (wave == 0) {
-    uint32_t mx = s_mx[0][lane];
-#pragma unroll
-    for (int w = 1; w < 4; ++w) mx = mx > s_mx[w][lane] ? mx : s_mx[w][lane];
-    if constexpr (kNorm) {
+    for (uint32_t i = wave; i < a.n_ssp; i += 4) ss += double(a.ssp[size_t(i) * kMaxPanel + tl]);
+    s_red[wave][lane] = ss;
+    __syncthreads();
+    if (wave == 0) {
       const float tot = float((s_red[0][lane] + s_red[1][lane]) + (s_red[2][lane] + s_red[3][lane]));
-      const float inv = 1.0f / sqrtf(tot / float(C) + a.eps);
-      s_inv[lane] = inv;
-      // the maximum of |x * gamma| * inv: (x * inv) * gamma rounds otherwise, by 2^-22 of it at most
-      mx = __float_as_uint(__uint_as_float(mx) * inv * (1.0f + 0x1p-20f));
+      s_inv[lane] = 1.0f / sqrtf(tot / float(C) + a.eps);
       // forwardDecode's break test (StepState::broken) on the token's input
       if (g == 0 && tok0 + lane < a.m &&
           ((a.chk == 1u && !isfinite(tot)) || (a.chk == 2u && !isfinite(a.x[size_t(tl) * C]))))
         a.brk[tl] = 1u;
     }
-    const float up = scale_up(mx, kUp);
-    s_up[lane] = up;
-    // (powers of two: exact; the codes enter the products times 16 or 64)
-    if (g == 0 && tok0 + lane < a.m)
-      a.down[tok0 + lane] = (BITS == 4 ? 0.0625f : BITS == 2 ? 0.015625f : 1.0f) / up;
+    __syncthreads();
   }
-  __syncthreads();
   const uint32_t T = a.tile;
 #pragma unroll
   for (uint32_t i = 0; i < 4; ++i) {
@@ -142,14 +101,21 @@ __global__ void __launch_bounds__(256) k_panel_split(PanelSplitArgs a) {
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[k] = (v[k] * inv) * gv[k];
     }
-    const float up = s_up[tok];
+    uint32_t mx = 0;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       if (t >= a.m) v[k] = 0.0f;
       s_x[ch * 8 + k][tok] = v[k];
+      const uint32_t b = __float_as_uint(v[k]) & 0x7fffffffu;
+      mx = mx > b ? mx : b;
     }
+    const float up = scale_up(lanes_umax<16>(mx), kUp);  // (the 16 lanes of a token)
     const bool in = t < a.n_tok;  // (not past the last token tile)
-    const size_t img = size_t(in ? t / T : 0u) * ng + g;
+    uint4* img = a.xs + (size_t(in ? t / T : 0u) * ng + g) * panel_image(T, BITS);
+    // (powers of two: exact; the codes enter the products times 16 or 64)
+    if (in && ch == 0)
+      reinterpret_cast<float*>(img + (panel_image(T, BITS) - kPanelScales / 4))[t % T] =
+          (BITS == 4 ? 0.0625f : BITS == 2 ? 0.015625f : 1.0f) / up;
     if constexpr (BITS == 16) {
       float h[8], l[8], r[8];
 #pragma unroll
@@ -160,14 +126,14 @@ __global__ void __launch_bounds__(256) k_panel_split(PanelSplitArgs a) {
         r[k] = (u - h[k]) - l[k];
       }
       if (!in) continue;
-      uint4* dst = a.xs + img * (T * 48) + (t % T) * 16 + (ch ^ (t & 15u));
+      uint4* dst = img + (t % T) * 16 + (ch ^ (t & 15u));
       dst[0] = make_uint4(pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7]));
       dst[T * 16] = make_uint4(pack2(l[0], l[1]), pack2(l[2], l[3]), pack2(l[4], l[5]), pack2(l[6], l[7]));
       dst[T * 32] = make_uint4(pack2(r[0], r[1]), pack2(r[2], r[3]), pack2(r[4], r[5]), pack2(r[6], r[7]));
     } else {
       uint32_t z[8], lo[4], hi[4];  // z: bytes, the balanced limbs of X
 #pragma unroll
-      for (int k = 0; k < 8; ++k) z[k] = (uint32_t(int(v[k] * up)) + 0x808080u) ^ 0x808080u;
+      for (int k = 0; k < 8; ++k) z[k] = (uint32_t(__float2int_rn(v[k] * up)) + 0x808080u) ^ 0x808080u;
       if constexpr (BITS == 2) {  // (as k_block_limbs: each of a pair sends the four values its neighbour needs)
         const bool odd = (ch & 1u) != 0;
         const uint32_t r0 = pair_u(odd ? z[0] : z[2], 1), r1 = pair_u(odd ? z[1] : z[3], 1);
@@ -184,7 +150,7 @@ __global__ void __launch_bounds__(256) k_panel_split(PanelSplitArgs a) {
         limb_words(z[1], z[3], z[5], z[7], hi);
       }
       if (!in) continue;
-      uint2* dst = reinterpret_cast<uint2*>(a.xs + img * (T * 32) + (t % T) * 8 + ((ch >> 1) ^ ((t >> 1) & 7u))) + (ch & 1u);
+      uint2* dst = reinterpret_cast<uint2*>(img + (t % T) * 8 + ((ch >> 1) ^ ((t >> 1) & 7u))) + (ch & 1u);
 #pragma unroll
       for (int L = 0; L < 4; ++L) dst[size_t(L) * T * 16] = make_uint2(lo[L], hi[L]);
     }
@@ -239,13 +205,23 @@ struct PanelRows {
     }
   }
 };
+// a group's image to LDS: XQ 16-byte pieces, the last kPanelScales / 4 of them in 4-byte loads, one a lane
 template <uint32_t XQ>
 __device__ __forceinline__ void panel_fetch(const uint4* src, uint4* dst, uint32_t wave, uint32_t lane) {
+  constexpr uint32_t P = XQ - kPanelScales / 4;
+  static_assert(P % 256 == 0 && kPanelScales == 256, "");
 #pragma unroll
-  for (uint32_t j = 0; j < XQ / 256; ++j) {
-    const uint32_t i0 = (wave * (XQ / 256) + j) * 64;
+  for (uint32_t j = 0; j < P / 256; ++j) {
+    const uint32_t i0 = (wave * (P / 256) + j) * 64;
     __builtin_amdgcn_global_load_lds(src + i0 + lane, dst + i0, 16, 0, 0);
   }
+  __builtin_amdgcn_global_load_lds(reinterpret_cast<const float*>(src + P) + wave * 64 + lane,
+                                   reinterpret_cast<float*>(dst + P) + wave * 64, 4, 0, 0);
+}
+// the factors of tokens 16 t + 4 q .. + 3 in an image
+template <uint32_t XQ>
+__device__ __forceinline__ f32x4_t panel_scale(const uint4* img, int t, uint32_t q) {
+  return __builtin_bit_cast(f32x4_t, img[XQ - kPanelScales / 4 + 4 * uint32_t(t) + q]);
 }
 template <int U, int TT>
 __device__ __forceinline__ void panel_store(const PanelGemmArgs& a, const PanelWork& p, const PanelRows<U>& R, uint32_t u0,
@@ -347,7 +323,7 @@ __device__ __forceinline__ void panel_loop_near(const PanelWork& p, uint4* x0, u
 // its row (4-bit: 16 bytes; 2-bit: 8).  The codes enter as bytes 16 (code - 8) (the nibble with its
 // top bit flipped is the two's complement; in the high half of the byte it is 16 times it) or 64 times
 // the 2-bit value: 4 (7) instructions for 8 (16) codes.  Per token tile and unit the four limbs' exact
-// sums, put together exactly in pairs (|D| <= 2^21) and scaled by the row's group scale.
+// sums, put together exactly in pairs (|D| <= 2^21) and scaled by the token's and the row's group scales.
 template <int BITS>
 struct PanelCodes {
   uint4 v[4];
@@ -359,14 +335,14 @@ struct PanelCodes<2> {
   uint32_t sc[4];
 };
 // One wave per SIMD with all the registers: the products of one (token tile, unit) step
-// alternate, one to three, with the vector instructions of the step before (order fixed by scheduling
-// barriers: left to itself the compiler puts the eight products first, then the 24 instructions),
+// alternate, one to three or four, with the vector instructions of the step before (order fixed by scheduling
+// barriers: left to itself the compiler puts the eight products first, then the 28 instructions),
 // and the next token tile's operands are read meanwhile.  (The file is built with the products'
 // results in vector registers: with 512 registers the compiler otherwise keeps them in accumulator
 // registers and copies each value out.  128 tokens spill.)
 template <int BITS, int TT>
 __global__ void __launch_bounds__(256, 1) k_panel_gemm(PanelGemmArgs a) {
-  constexpr uint32_t T = 16 * TT, XQ = T * 32;  // 16-byte pieces of one group's token tile
+  constexpr uint32_t T = 16 * TT, XQ = panel_image(T, BITS);  // 16-byte pieces of one group's token tile
   __shared__ __align__(16) uint4 s_x0[XQ], s_x1[XQ];
   const uint32_t tid = threadIdx.x, lane = tid & 63, n = lane & 15, q = lane >> 4;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -394,12 +370,14 @@ __global__ void __launch_bounds__(256, 1) k_panel_gemm(PanelGemmArgs a) {
   const uint32_t a0 = n * 8 + ((2 * q) ^ (n >> 1)), a1 = n * 8 + ((2 * q + 1) ^ (n >> 1));
   auto compute = [&](const uint4* xsrc, const PanelCodes<BITS>& c) {
     i32x4_t B[4][2], A[2][4][2], D[2][4];
+    f32x4_t ts[2];
     float sc[4];
     auto read = [&](int t, int L, int s) {
       A[t & 1][L][s] = __builtin_bit_cast(i32x4_t, xsrc[uint32_t(L) * (T * 8) + uint32_t(t) * 128 + (s ? a1 : a0)]);
     };
 #pragma unroll
     for (int k = 0; k < 8; ++k) read(0, k & 3, k >> 2);
+    ts[0] = panel_scale<XQ>(xsrc, 0, q);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
 #pragma unroll
@@ -427,29 +405,32 @@ __global__ void __launch_bounds__(256, 1) k_panel_gemm(PanelGemmArgs a) {
           const int L = k & 3, s = k >> 2;
           D[b][L] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[t & 1][L][s], B[u][s], s ? D[b][L] : i32x4_t{0, 0, 0, 0}, 0, 0, 0);
         }
-        if (fin) {  // 24 instructions in eight threes, the limbs' sums in the order they complete
+        if (fin) {  // 28 instructions in eight threes and fours, the limbs' sums in the order they complete
           const i32x4_t(&E)[4] = D[b ^ 1];
 #define CHPE_LO(j) lo[j] = E[0][j] + int(uint32_t(E[1][j]) << 8)
 #define CHPE_HI(j) hi[j] = E[2][j] + int(uint32_t(E[3][j]) << 8)
 #define CHPE_F(j) fh[j] = fmaf(fh[j], 65536.0f, fl[j])
+#define CHPE_S(j) fh[j] *= ts[tp & 1][j]
 #define CHPE_ACC(j) acc[up][tp][j] = fmaf(fh[j], sc[up], acc[up][tp][j])
-          if (k == 0) CHPE_LO(0), CHPE_LO(1), CHPE_LO(2);
-          if (k == 1) CHPE_LO(3), fl[0] = float(lo[0]), fl[1] = float(lo[1]);
-          if (k == 2) fl[2] = float(lo[2]), fl[3] = float(lo[3]), CHPE_HI(0);
-          if (k == 3) CHPE_HI(1), CHPE_HI(2), CHPE_HI(3);
-          if (k == 4) fh[0] = float(hi[0]), fh[1] = float(hi[1]), fh[2] = float(hi[2]);
-          if (k == 5) fh[3] = float(hi[3]), CHPE_F(0), CHPE_F(1);
-          if (k == 6) CHPE_F(2), CHPE_F(3), CHPE_ACC(0);
-          if (k == 7) CHPE_ACC(1), CHPE_ACC(2), CHPE_ACC(3);
+          if (k == 0) CHPE_LO(0), CHPE_LO(1), CHPE_LO(2), CHPE_LO(3);
+          if (k == 1) fl[0] = float(lo[0]), fl[1] = float(lo[1]), fl[2] = float(lo[2]);
+          if (k == 2) fl[3] = float(lo[3]), CHPE_HI(0), CHPE_HI(1);
+          if (k == 3) CHPE_HI(2), CHPE_HI(3), fh[0] = float(hi[0]), fh[1] = float(hi[1]);
+          if (k == 4) fh[2] = float(hi[2]), fh[3] = float(hi[3]), CHPE_F(0);
+          if (k == 5) CHPE_F(1), CHPE_F(2), CHPE_F(3), CHPE_S(0);
+          if (k == 6) CHPE_S(1), CHPE_S(2), CHPE_S(3);
+          if (k == 7) CHPE_ACC(0), CHPE_ACC(1), CHPE_ACC(2), CHPE_ACC(3);
 #undef CHPE_LO
 #undef CHPE_HI
 #undef CHPE_F
+#undef CHPE_S
 #undef CHPE_ACC
         }
         if (mul && t + 1 < TT && (k & 3) == 1) {  // two reads of the next tile per step
           const int r = 2 * u + (k >> 2);
           read(t + 1, r & 3, r >> 2);
         }
+        if (mul && t + 1 < TT && u == 1 && k == 2) ts[(t + 1) & 1] = panel_scale<XQ>(xsrc, t + 1, q);  // (the tile before t is done)
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -473,7 +454,7 @@ __global__ void __launch_bounds__(256, 1) k_panel_gemm(PanelGemmArgs a) {
 
 // fp16 weights: v_mfma_f32_16x16x32_f16, D lane (n, q) = row n, tokens 4 q .. + 3; the k slots of step
 // d hold columns 32 q + 8 d .. + 7.  The products are exact; the small parts have a sum of their own, each
-// step of 16 columns of the high parts has one, and those are added up in 64 bits (measured on random
+// step of 16 columns of the high parts has one, and those are scaled and added up in 64 bits (measured on random
 // weights, 128 columns: 0.74 x 2^-24 of the sum, against 1.29 in one chain).  U = 2 units per wave:
 // 64 bytes of codes per lane, unit and group.
 // The small parts' sum is not the starting value of the first 16 columns' product: that is another opcode, and
@@ -485,7 +466,7 @@ struct PanelHalves {
 };
 __global__ void __launch_bounds__(256, 2) k_panel_gemm_h(PanelGemmArgs a) {
   constexpr int U = 2, TT = 2;
-  constexpr uint32_t T = 16 * TT, XQ = T * 48;
+  constexpr uint32_t T = 16 * TT, XQ = panel_image(T, 16);
   __shared__ __align__(16) uint4 s_x0[XQ], s_x1[XQ];
   const uint32_t tid = threadIdx.x, lane = tid & 63, n = lane & 15, q = lane >> 4;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -511,7 +492,9 @@ __global__ void __launch_bounds__(256, 2) k_panel_gemm_h(PanelGemmArgs a) {
     auto operand = [&](int part, int d, int t) {
       return as_half8(xsrc[uint32_t(part) * (T * 16) + uint32_t(t) * 256 + n * 16 + ((4 * q + uint32_t(d)) ^ n)]);
     };
-    f32x4_t D[U][TT];
+    f32x4_t D[U][TT], ts[TT];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) ts[t] = panel_scale<XQ>(xsrc, t, q);
 #pragma unroll
     for (int part = 2; part >= 1; --part)
 #pragma unroll
@@ -537,7 +520,7 @@ __global__ void __launch_bounds__(256, 2) k_panel_gemm_h(PanelGemmArgs a) {
           const f32x4_t E0 = __builtin_amdgcn_mfma_f32_16x16x16f16(A0, B0, z, 0, 0, 0);
           const f32x4_t E1 = __builtin_amdgcn_mfma_f32_16x16x16f16(A1, B1, z, 0, 0, 0);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[u][t][j] += double(E0[j]) + double(E1[j]);
+          for (int j = 0; j < 4; ++j) acc[u][t][j] = fma(double(E0[j]) + double(E1[j]), double(ts[t][j]), acc[u][t][j]);
         }
       }
 #pragma unroll
@@ -545,7 +528,7 @@ __global__ void __launch_bounds__(256, 2) k_panel_gemm_h(PanelGemmArgs a) {
 #pragma unroll
       for (int t = 0; t < TT; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[u][t][j] += double(D[u][t][j]);
+        for (int j = 0; j < 4; ++j) acc[u][t][j] = fma(double(D[u][t][j]), double(ts[t][j]), acc[u][t][j]);
   };
   panel_loop_near<PanelHalves>(p, s_x0, s_x1, issue, fetch, compute);
   f32x4_t sum[U][TT];
@@ -564,7 +547,7 @@ __global__ void __launch_bounds__(256, 2) k_panel_gemm_h(PanelGemmArgs a) {
 // The ranges' sums of the OPW rows in flight together; then the rows' packed correction entries,
 // which are one consecutive run: 64 entries in one load, one per lane, and 16 columns' loads in
 // flight at a time, whatever row they belong to (row by row, with an entry load and a column load
-// chain each, the SwiGLU launch of the 72B model at 300 tokens took 409 us, of which 75 the contended maxima below; this way 98).  Then
+// chain each, the SwiGLU launch of the 72B model at 300 tokens took 334 us; this way EPI_US).  Then
 // through LDS to outputs-fastest order for the writes.  Bound by the corrections' reads (4 bytes
 // per entry and token, from L2) and the partial sums.
 template <int MODE, int OPW>
@@ -578,7 +561,6 @@ __global__ void __launch_bounds__(256) k_panel_epi(PanelEpiArgs a) {
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t tok0 = blockIdx.y * 64, m = a.m, half = a.head_dim / 2;
   const uint32_t tl = tok0 + lane < m ? tok0 + lane : m - 1;
-  const float down = a.down[tl];
   const size_t rstride = size_t(a.rows_all) * a.n_tok;
   // output o -> part and row (the first of its pair); OPW outputs from a multiple of OPW are
   // consecutive rows (the parts' outputs and half are multiples of 8)
@@ -616,7 +598,7 @@ __global__ void __launch_bounds__(256) k_panel_epi(PanelEpiArgs a) {
 #pragma unroll
         for (int i = 0; i < OPW; ++i) s[i] += double(ps[rg * rstride + size_t(i) * a.n_tok]);
 #pragma unroll
-      for (int i = 0; i < OPW; ++i) s_o[k][lane][wave * OPW + i] = float(s[i]) * down;  // (a power of two: exact)
+      for (int i = 0; i < OPW; ++i) s_o[k][lane][wave * OPW + i] = float(s[i]);
       const uint32_t eb = __builtin_amdgcn_readlane(off, 0), ee = __builtin_amdgcn_readlane(off, OPW);
       float c = 0.0f;
       uint32_t row = 0, bound = __builtin_amdgcn_readlane(off, 1);
@@ -653,29 +635,19 @@ __global__ void __launch_bounds__(256) k_panel_epi(PanelEpiArgs a) {
     const bool ok = t < m && o < a.total;
     if constexpr (kAcc) {
       float sq = 0.0f;
-      uint32_t mx = 0;
       if (ok) {
         float* y = a.part[0].y + size_t(t) * a.part[0].rows + o;
         const bool upd = o < a.part[0].wrows && a.brk[t] == 0u;  // rows past the tiles and broken tokens stay
         const float yo = *y, yn = upd ? yo + s_o[0][tok][oi] : yo;
         if (upd) *y = yn;
         sq = yn * yn;
-        mx = __float_as_uint(yn * a.gamma_next[o]) & 0x7fffffffu;
       }
 #pragma unroll
       for (int x = 1; x < int(TILE); x <<= 1) sq = pair_sum(sq, x);
-      mx = lanes_umax<int(TILE)>(mx);
-      if (oi == 0 && t < m) {
-        a.ssp_out[size_t(blockIdx.x) * kMaxPanel + t] = sq;
-        a.mx_out[size_t(blockIdx.x) * kMaxPanel + t] = mx;
-      }
+      if (oi == 0 && t < m) a.ssp_out[size_t(blockIdx.x) * kMaxPanel + t] = sq;
     } else if constexpr (kSwi) {
       const float g = s_o[0][tok][oi];
-      const float y = ok ? g / (1.0f + expf(-g)) * s_o[1][tok][oi] : 0.0f;  // silu(g)*u: :159-161, :1746-1748
-      if (ok) a.part[0].y[size_t(t) * a.part[0].rows + o] = y;
-      uint32_t mx = __float_as_uint(y) & 0x7fffffffu;
-      mx = lanes_umax<int(TILE)>(mx);
-      if (oi == 0 && t < m) atomicMax(&a.tokmax_out[(blockIdx.x % kPanelMaxSlots) * kMaxPanel + t], mx);
+      if (ok) a.part[0].y[size_t(t) * a.part[0].rows + o] = g / (1.0f + expf(-g)) * s_o[1][tok][oi];  // silu(g)*u: :159-161, :1746-1748
     } else if constexpr (kRope) {
 #pragma clang fp contract(off)
       if (!ok) continue;
@@ -764,7 +736,6 @@ __device__ __forceinline__ void panel_attn_out(const PanelAttnArgs& a, const f32
     f[w] = s_l[w][row] == 0.0f ? 0.0f : expf(s_m[w][row] - M);
     L = fmaf(s_l[w][row], f[w], L);
   }
-  uint32_t mx = 0;
 #pragma unroll
   for (int i = 0; i < HD / 64; ++i) {
 #pragma clang fp contract(off)
@@ -786,14 +757,7 @@ __device__ __forceinline__ void panel_attn_out(const PanelAttnArgs& a, const f32
     }
     if (t < a.m)
       *reinterpret_cast<float4*>(a.out + (size_t(t) * a.H + head) * HD + d) = make_float4(v[0], v[1], v[2], v[3]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t b = __float_as_uint(v[j]) & 0x7fffffffu;
-      mx = mx > b ? mx : b;
-    }
   }
-  mx = lanes_umax<16>(mx);
-  if (c == 0 && t < a.m) atomicMax(&a.tokmax_out[(head % kPanelMaxSlots) * kMaxPanel + t], mx);
 }
 
 template <int HD, int G>
@@ -1031,12 +995,8 @@ __global__ void __launch_bounds__(256) k_panel_attn_f(PanelAttnArgs a) {
 
 }  // namespace
 
-void launch_panel_begin(const PanelBeginArgs& a, hipStream_t st) {
-  launch_kernel(&k_panel_begin, dim3((a.n_max + 255) / 256), dim3(256), st, a);
-}
-
-void launch_panel_rowmax(const float* x, const float* gamma, uint32_t C, uint32_t m, uint32_t* mx_out, hipStream_t st) {
-  launch_kernel(&k_panel_rowmax, dim3(m), dim3(256), st, x, gamma, C, mx_out);
+void launch_panel_begin(StepState* state, uint32_t token, uint32_t pos, hipStream_t st) {
+  launch_kernel(&k_panel_begin, dim3(1), dim3(1), st, state, token, pos);
 }
 
 void launch_panel_split(const PanelSplitArgs& a, uint32_t bits, hipStream_t st) {

@@ -18,6 +18,7 @@ import numpy as np
 import pytest
 
 import chpe_amd as ca
+import oracle as orc
 from conftest import archive_path
 
 pytestmark = pytest.mark.gpu
@@ -78,7 +79,6 @@ def test_panel_break(w4_archive, monkeypatch):
     """forwardDecode's non-finite break (StepState::broken) in a panel: an infinite outlier weight
     in layer 1's down projection stops every token after that layer; the final norm and the LM head
     see that hidden state, as in the decode steps."""
-    import oracle as orc
     from test_gpu_nonfinite import inf_outlier_edit
     li = orc.layer_info(1, 1)
     off, b = inf_outlier_edit(w4_archive, li["down_proj"], li["down_tiles"])
@@ -141,6 +141,52 @@ def test_panel_nonfinite_row(kind, arch, vocab, kv16, at, bar, monkeypatch):
             d = rel(nxt[1][fin], nxt[0][fin])
             print(f"arch {arch} kv16 {kv16}: the step at {at}: {d:.2e}", flush=True)
             assert d <= bar
+        finally:
+            e.close()
+            steps.close()
+    finally:
+        os.unlink(path)
+
+
+@pytest.mark.timeout(300)
+@pytest.mark.parametrize("kind,gain", [(ca.PACK_3B_W4, 2.0 ** 16), (ca.PACK_3B_FP16_RAW, 2.0 ** 24)])
+def test_panel_outlier_channel(kind, gain, monkeypatch):
+    """One channel of every normalised input `gain` times the others, as the massive activations of real
+    models: the other channels keep their bits, since every 128-column group has a scale of its own
+    in the panels as in the decode steps.  (The weights of the channel's own group are zero in every
+    projection that reads a normalised input, so the results depend on the other groups alone; with a
+    scale per token the logits are 1e-3 apart.)"""
+    src, raw, c0 = archive_path(kind), kind == ca.PACK_3B_FP16_RAW, 640
+    fd, path = tempfile.mkstemp(suffix=".chpe", prefix="qwen2.5-3b-mod-", dir=os.path.dirname(str(src)))
+    os.close(fd)
+    shutil.copyfile(src, path)
+    try:
+        b = np.memmap(path, dtype=np.uint8, mode="r+")
+        stride = 16384 if raw else 17408
+        for l in range(36):
+            li = orc.layer_info(0 if raw else 1, l)
+            for name in ("q", "k", "v", "gate", "up"):
+                rec, n = li[name + "_proj"], li[name + "_tiles"]
+                t = b[4096 + rec * stride:4096 + (rec + n) * stride].reshape(n, stride)
+                if raw:
+                    t.view(np.float16).reshape(-1, 2048)[:, c0:c0 + 128] = 0
+                    continue
+                t[:, 64:16448].reshape(n, 16, 1024)[:, :, c0 // 2:c0 // 2 + 64] = 0x88
+                cols = t[:, 16448 + 816:16448 + 832].copy().view(np.uint16)
+                vals = t[:, 16448 + 560:16448 + 816].copy().view(np.float16).reshape(n, 16, 8)
+                vals[np.broadcast_to((cols // 128 == c0 // 128)[:, None], vals.shape)] = 0
+                t[:, 16448 + 560:16448 + 816] = vals.reshape(n, 128).view(np.uint8)
+            for rec in (li["input_norm"], li["post_norm"]):
+                at = 4096 + rec * stride + (0 if raw else 64) + 4 * (c0 + 77)
+                b[at:at + 4] = (b[at:at + 4].copy().view(np.float32) * np.float32(gain)).view(np.uint8)
+        b.flush()
+        del b
+        e, steps = engines(path, 0, 80, False, monkeypatch)
+        try:
+            toks = np.random.default_rng(5).integers(0, 151936, 70).astype(np.uint32)
+            want, got = (x.forward_tokens(toks, want_logits=True)[1] for x in (steps, e))
+            print(f"kind {kind} outlier channel: logits {rel(got, want):.2e}", flush=True)
+            assert np.isfinite(want).all() and rel(got, want) <= 4e-5
         finally:
             e.close()
             steps.close()
