@@ -244,7 +244,9 @@ __device__ __forceinline__ void panel_store(const PanelGemmArgs& a, const PanelW
 // them); past the last group the last one's codes are loaded again, not used.  The barrier is
 // a bare s_barrier behind a wait for the token tile alone: the only loads younger than it are
 // one group's codes (kCodeLoads of them, the order fixed by the scheduling barriers), and for the
-// wave's own reads of the buffer that is overwritten next.
+// wave's own reads of the buffer that is overwritten next.  The wait is right only if the compiler issues
+// at least kCodeLoads vector loads between a tile's and the next wait: one per unit's codes and one per unit's
+// scale here (tests/test_panel_isa.py checks every path of every instance).
 constexpr int kCodeLoads = 8;
 template <class Codes, class Issue, class Fetch, class Compute, class Fold>
 __device__ __forceinline__ void panel_loop(const PanelWork& p, uint4* x0, uint4* x1, const Issue& issue, const Fetch& fetch,
@@ -339,7 +341,8 @@ struct PanelCodes<2> {
 // barriers: left to itself the compiler puts the eight products first, then the 28 instructions),
 // and the next token tile's operands are read meanwhile.  (The file is built with the products'
 // results in vector registers: with 512 registers the compiler otherwise keeps them in accumulator
-// registers and copies each value out.  128 tokens spill.)
+// registers and copies each value out.  Tiles of 80 tokens and more spill two to four registers, once
+// in four groups; 128 tokens spill in every group.)
 template <int BITS, int TT>
 __global__ void __launch_bounds__(256, 1) k_panel_gemm(PanelGemmArgs a) {
   constexpr uint32_t T = 16 * TT, XQ = panel_image(T, BITS);  // 16-byte pieces of one group's token tile

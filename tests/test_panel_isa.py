@@ -3,7 +3,10 @@ source relies on and cannot state:
 
 * k_panel_gemm_h: no product takes as its starting sum the result of a product of another opcode.  The compiler puts
   no wait between two products that hand on exactly the same registers; across opcodes the second
-  one can take the sum before the first one's result is there."""
+  one can take the sum before the first one's result is there.
+* k_panel_gemm: the barrier before a token tile's use waits until at most kCodeLoads vector loads are outstanding;
+  that is the tile only if at least that many loads follow it.  Every path from a tile's last load into LDS
+  to the next wait issues them, or the wait is for all loads."""
 import re
 import shlex
 import subprocess
@@ -61,3 +64,57 @@ def test_products_start_from_their_own_opcode(kernels):
             elif t.startswith("v_") and " v[" in t:
                 last.pop(t.split()[1].rstrip(","), None)
         assert n > 0, name
+
+
+def waits_after(ins, start):
+    """(loads issued since, outstanding allowed) at the next vector-memory wait on every path from `start`"""
+    labels = {t[:-1]: i for i, t in enumerate(ins) if t.endswith(":")}
+    found, seen, todo = [], set(), [(start, 0)]
+    while todo:
+        i, n = todo.pop()
+        while i < len(ins) and (i, n) not in seen:
+            seen.add((i, n))
+            t = ins[i]
+            m = re.search(r"vmcnt\((\d+)\)", t)
+            if m:
+                found.append((n, int(m.group(1))))
+                break
+            if "load_lds" in t:  # (the next tile's loads before any wait for this one)
+                found.append((n, 63))
+                break
+            n += t.startswith(("global_load", "scratch_load"))
+            if t.startswith("s_branch"):
+                i = labels[t.split()[1]]
+                continue
+            if t.startswith("s_cbranch"):
+                todo.append((labels[t.split()[1]], n))
+            if t.startswith("s_endpgm"):
+                found.append((n, 63))
+                break
+            i += 1
+    return found
+
+
+@pytest.mark.timeout(600)
+def test_tile_waits_have_their_loads(kernels):
+    src = (ca.PKG_DIR / "csrc" / "panel.hip").read_text()
+    allowed = int(re.search(r"kCodeLoads = (\d+);", src).group(1))
+    found = of(kernels, "k_panel_gemmI")
+    assert len(found) == 10
+    for name, ins in found.items():
+        tiles = [i for i, t in enumerate(ins) if "load_lds" in t and not any("load_lds" in x for x in between(ins, i))]
+        assert len(tiles) >= 6, name  # the first tile, four groups per trip, the remainders
+        waits = [w for i in tiles for w in waits_after(ins, i + 1)]
+        assert any(limit == allowed for _, limit in waits), name
+        for n, limit in waits:
+            assert limit == 0 or (limit <= allowed and n >= limit), (name, n, limit)
+
+
+def between(ins, i):
+    """the instructions from i to the next wait, barrier, load or branch"""
+    for t in ins[i + 1:]:
+        if t.startswith(("s_waitcnt", "s_barrier", "s_cbranch", "s_branch", "s_endpgm", "global_load_dword", "global_load_u")):
+            if "load_lds" in t:
+                yield t
+            return
+        yield t
