@@ -487,16 +487,17 @@ __global__ void __launch_bounds__(256) k_dn_gnorm_block(DnBlockArgs a) {
 
 }  // namespace
 
-void launch_dn_block(const DnBlockArgs& a, hipStream_t st) {
+bool launch_dn_block(const DnBlockArgs& a, hipStream_t st) {
   // (the engine plans the 9B layers: 4 taps, 128-wide heads, an even number of value heads in eights)
   if (a.taps != kDnConvTaps || a.head_dim != 128 || a.n_v_heads % 8 || a.n_v_heads % a.n_k_heads ||
       a.channels != (2 * a.n_k_heads + a.n_v_heads) * 128 || a.channels > a.n_v_heads * 8 * 256) {
     std::fprintf(stderr, "chpe: the multi-token DeltaNet kernels are built for the 9B layers\n");
-    return;
+    return false;
   }
   launch_kernel(&k_dn_prep, dim3(a.n_k_heads + a.n_v_heads / 2, a.m), dim3(256), st, a);
   launch_kernel(&k_dn_scan, dim3(a.n_v_heads, 8), dim3(256), st, a);
   launch_kernel(&k_dn_gnorm_block, dim3(a.n_v_heads / 8, a.m), dim3(256), st, a);
+  return true;
 }
 
 bool deltanet_supported(uint32_t n_v_heads, uint32_t n_k_heads, uint32_t head_dim, uint32_t taps) {

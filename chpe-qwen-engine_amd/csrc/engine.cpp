@@ -1218,7 +1218,7 @@ uint32_t Engine::enqueue_block_gemv(const ProjPlan* const* parts, float* const* 
     b.cpack[i] = gp.corr ? p.bpack : nullptr;
     b.coff[i] = gp.corr ? p.boff : nullptr;
     if (gp.corr && !p.boff) {  // (every block-step part's table has its packed form: plan_projection, plan_block)
-      bpart_short_ = true;
+      not_built_ = true;
       return 1;
     }
     gp.rope_role = mode == GemvMode::QkvRope ? (roles_in ? roles_in[i] : roles[i]) : 0u;
@@ -1234,7 +1234,7 @@ uint32_t Engine::enqueue_block_gemv(const ProjPlan* const* parts, float* const* 
   b.partial = d_bpartial_;
   b.brk = d_bbrk_;
   if (size_t(block_gemv_ranges(units, C, m)) * b.rows_all * kMaxBlock > bpart_floats_) {  // (the plan's sizes)
-    bpart_short_ = true;
+    not_built_ = true;
     return 1;
   }
   if (mode == GemvMode::QkvRope) {
@@ -1270,9 +1270,10 @@ int Engine::block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t
     hipGraphExec_t& ge = bgraph_exec_[m];
     if (!ge) {
       if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) != hipSuccess) return -3;
+      not_built_ = false;
       record_block(mm, st);
       if (hipStreamEndCapture(st, &g) != hipSuccess) return -3;
-      if (bpart_short_) {
+      if (not_built_) {
         (void)hipGraphDestroy(g);
         g = nullptr;
         return -3;
@@ -1281,8 +1282,9 @@ int Engine::block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t
     }
     if (hipGraphLaunch(ge, st) != hipSuccess) return -3;
   } else {
+    not_built_ = false;
     record_block(mm, st);
-    if (bpart_short_) {
+    if (not_built_ || hipGetLastError() != hipSuccess) {
       (void)hipStreamSynchronize(st);
       return -3;
     }
@@ -1438,7 +1440,7 @@ void Engine::record_block_hybrid(uint32_t mm, hipStream_t st) {
         float* outb[1] = {d_bhx3_};
         enqueue_block_gemv(inb, outb, 1, GemvMode::QkvRope, d_bx_, D, L.gamma_in, n_ss, mm, l, st, store, 32);
       }
-      launch_dn_block(dn_block_args(l, d_bhx0_, d_bhx1_, d_bhx2_, d_bhx3_, d_bhconv_, d_battn_, d_bbrk_, mm), st);
+      if (!launch_dn_block(dn_block_args(l, d_bhx0_, d_bhx1_, d_bhx2_, d_bhx3_, d_bhconv_, d_battn_, d_bbrk_, mm), st)) not_built_ = true;
     }
     const ProjPlan* o[1] = {&Hy.out};
     n_ss = enqueue_block_gemv(o, hid, 1, GemvMode::Accum, d_battn_, 4096, nullptr, 0, mm, l, st);
@@ -1535,6 +1537,10 @@ uint32_t Engine::enqueue_panel_gemm(const ProjPlan* const* parts, float* const* 
   }
   const uint32_t rows_all = 16 * units;
   const PanelShape sh = panel_shape(units, ng, m, bits, ppart_floats_);
+  if (sh.tile == 0) {
+    not_built_ = true;
+    return 1;
+  }
   const uint32_t n_tok = sh.ntt * sh.tile;  // (< m + 112: within the buffers' kPanelRows rows)
   PanelSplitArgs s{};
   s.x = x;
@@ -1562,7 +1568,7 @@ uint32_t Engine::enqueue_panel_gemm(const ProjPlan* const* parts, float* const* 
   g.ranges = sh.ranges;
   g.xs = d_pxs_;
   g.partial = d_ppart_;
-  launch_panel_gemm(g, bits, sh.tile, st);
+  if (!launch_panel_gemm(g, bits, sh.tile, st)) not_built_ = true;
   e.n_parts = n;
   e.m = m;
   e.n_tok = n_tok;
@@ -1635,7 +1641,7 @@ void Engine::enqueue_panel(uint32_t token, uint32_t pos, uint32_t m, hipStream_t
           enqueue_panel_gemm(inb, outb, 1, GemvMode::QkvRope, d_px_, D, L.gamma_in, n_ss, m, pos, l, st,
                              store, 32);
         }
-        launch_dn_block(dn_block_args(l, d_phx0_, d_phx1_, d_phx2_, d_phx3_, d_phconv_, d_pattn_, d_pbrk_, m), st);
+        if (!launch_dn_block(dn_block_args(l, d_phx0_, d_phx1_, d_phx2_, d_phx3_, d_phconv_, d_pattn_, d_pbrk_, m), st)) not_built_ = true;
       }
       const ProjPlan* o[1] = {&Hy.out};
       n_ss = enqueue_panel_gemm(o, hid, 1, GemvMode::Accum, d_pattn_, 4096, nullptr, 0, m, pos, l, st);
@@ -1653,6 +1659,7 @@ int Engine::prompt_forward(const uint32_t* tokens, size_t n, ForwardResult* out)
   hipStream_t st = stream_;
   if (hipMemcpyAsync(d_prompt_, tokens, n * 4, hipMemcpyHostToDevice, st) != hipSuccess) return -3;
   if (cfg_.hybrid) reset_hybrid_state(st);  // a new sequence
+  not_built_ = false;
   // equal panels
   const size_t np = (n + kMaxPanel - 1) / kMaxPanel, per = (n + np - 1) / np;
   size_t m = 0;
@@ -1670,6 +1677,10 @@ int Engine::prompt_forward(const uint32_t* tokens, size_t n, ForwardResult* out)
       hipMemcpyAsync(d_hidden_, last, arch_.hidden_dim * 4, hipMemcpyDeviceToDevice, st) != hipSuccess)
     return -3;
   enqueue_head(last, st);
+  if (not_built_ || hipGetLastError() != hipSuccess) {  // (a launch that was refused: the synchronisation does not say so)
+    (void)hipStreamSynchronize(st);
+    return -3;
+  }
   if (hipMemcpyAsync(h_result_, d_result_, sizeof(StepResult), hipMemcpyDeviceToHost, st) != hipSuccess) return -3;
   if (sync()) return -3;
   out->argmax_token = h_result_->argmax;

@@ -317,7 +317,7 @@ class Engine {
   float *d_bx_ = nullptr, *d_bq_ = nullptr, *d_battn_ = nullptr, *d_bmlp_ = nullptr, *d_blog_ = nullptr;
   float *d_bpartial_ = nullptr, *d_bpml_ = nullptr, *d_bpacc_ = nullptr;
   size_t bpart_floats_ = 0;   // d_bpartial_'s capacity
-  bool bpart_short_ = false;  // a block GEMV's partial sums did not fit (not launched; the block step fails)
+  bool not_built_ = false;    // a launcher refused its shape (nothing launched): the block step or the panel fails
   float* d_bss_ = nullptr;  // [kMaxSsPartials][kMaxBlock]: Σx² partials of the hidden rows for the next norm
   // the hybrid's block activations, [kMaxBlock][rows]: the in-projections' outputs (as d_hx0_ ..
   // d_hx3_) and the conv outputs

@@ -409,7 +409,7 @@ struct DnBlockArgs {
   float eps;
   const uint32_t* brk;      // [m]: token t broke before this layer (its state updates are skipped)
 };
-void launch_dn_block(const DnBlockArgs& a, hipStream_t stream);
+bool launch_dn_block(const DnBlockArgs& a, hipStream_t stream);  // false: a shape that is not built, nothing launched
 
 // The hybrid model's gated full-attention layer around the decode attention kernels
 // (transformers' Qwen3_5Attention): per query head the RMS norm (q_norm gains) and the rotary
@@ -514,11 +514,11 @@ struct PanelAttnArgs {
 };
 void launch_panel_begin(StepState* state, uint32_t token, uint32_t pos, hipStream_t stream);  // the panel's first position
 void launch_panel_split(const PanelSplitArgs& a, uint32_t bits, hipStream_t stream);
-void launch_panel_gemm(const PanelGemmArgs& a, uint32_t bits, uint32_t tile, hipStream_t stream);
+bool launch_panel_gemm(const PanelGemmArgs& a, uint32_t bits, uint32_t tile, hipStream_t stream);  // false: a tile that is not built
 void launch_panel_epi(const PanelEpiArgs& a, GemvMode mode, hipStream_t stream);
 void launch_panel_attention(const PanelAttnArgs& a, hipStream_t stream);
 uint32_t panel_epi_tile(uint32_t total, uint32_t m);  // outputs per epilogue workgroup
-// how a GEMM of n_units units, ng groups and m tokens is cut up (at most max_partials partial sums)
+// how a GEMM of n_units units, ng groups and m tokens is cut up (at most max_partials partial sums; tile 0: too few)
 struct PanelShape {
   uint32_t tile, ntt, nrt, ranges;  // tokens per tile, token tiles, row tiles, column ranges
 };

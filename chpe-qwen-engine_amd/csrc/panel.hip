@@ -1039,21 +1039,26 @@ PanelShape panel_shape(uint32_t n_units, uint32_t ng, uint32_t m, uint32_t bits,
 }
 
 template <int BITS>
-void launch_panel_gemm_of(const PanelGemmArgs& a, uint32_t tile, dim3 grid, hipStream_t st) {
+bool launch_panel_gemm_of(const PanelGemmArgs& a, uint32_t tile, dim3 grid, hipStream_t st) {
   switch (tile) {
     case 32: launch_kernel(&k_panel_gemm<BITS, 2>, grid, dim3(256), st, a); break;
     case 64: launch_kernel(&k_panel_gemm<BITS, 4>, grid, dim3(256), st, a); break;
     case 80: launch_kernel(&k_panel_gemm<BITS, 5>, grid, dim3(256), st, a); break;
     case 96: launch_kernel(&k_panel_gemm<BITS, 6>, grid, dim3(256), st, a); break;
     case 112: launch_kernel(&k_panel_gemm<BITS, 7>, grid, dim3(256), st, a); break;
+    default: return false;
   }
+  return true;
 }
 
-void launch_panel_gemm(const PanelGemmArgs& a, uint32_t bits, uint32_t tile, hipStream_t st) {
+bool launch_panel_gemm(const PanelGemmArgs& a, uint32_t bits, uint32_t tile, hipStream_t st) {
   const dim3 grid(a.nrt * a.ntt * a.ranges);
-  if (bits == 16) launch_kernel(&k_panel_gemm_h, grid, dim3(256), st, a);
-  else if (bits == 2) launch_panel_gemm_of<2>(a, tile, grid, st);
-  else launch_panel_gemm_of<4>(a, tile, grid, st);
+  if (bits == 16) {
+    if (tile != 32) return false;
+    launch_kernel(&k_panel_gemm_h, grid, dim3(256), st, a);
+    return true;
+  }
+  return bits == 2 ? launch_panel_gemm_of<2>(a, tile, grid, st) : launch_panel_gemm_of<4>(a, tile, grid, st);
 }
 
 // outputs per workgroup: 32, or 16 where that leaves the CUs short of workgroups

@@ -10,6 +10,7 @@ rounding boundary are stored one fp16 step apart (2^-11 of the value): measured 
 bars four times that.  An argmax may differ only where the two best logits are closer
 than the bar.  (The 72B archives' panels: test_gpu_models.py, a prompt of 11 against the block step
 and the oracle.)"""
+import ctypes
 import os
 import shutil
 import tempfile
@@ -192,3 +193,22 @@ def test_panel_outlier_channel(kind, gain, monkeypatch):
             steps.close()
     finally:
         os.unlink(path)
+
+
+@pytest.mark.parametrize("call,n", [("forward_tokens", 3), ("forward_tokens", 20), ("prefill", 40)])
+def test_refused_launch_is_an_error(w4_archive, call, n):
+    """An error on the calling thread when the launches are done, as a refused launch leaves one (here: a device
+    that does not exist), fails the call that it belongs to, in panels as in decode steps (n = 3); the call after it
+    is right again."""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    toks = np.random.default_rng(n).integers(0, 151936, n).astype(np.uint32)
+    e = ca.Engine(w4_archive, arch=0, max_seq_len=64, kv_f16=False)
+    try:
+        want = getattr(e, call)(toks, want_logits=True)[1]
+        assert hip.hipSetDevice(9999) != 0
+        with pytest.raises(ca.EngineError):
+            getattr(e, call)(toks)
+        got = getattr(e, call)(toks, want_logits=True)[1]
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    finally:
+        e.close()
