@@ -78,10 +78,11 @@ std::unique_ptr<Engine> Engine::create(const uint8_t* bytes, size_t len, const E
 
 Engine::~Engine() {
   if (stream_) (void)hipStreamSynchronize(stream_);
-  for (uint32_t m = 0; m <= kMaxBlock; ++m) {
-    if (bgraph_exec_[m]) (void)hipGraphExecDestroy(bgraph_exec_[m]);
-    if (bgraph_[m]) (void)hipGraphDestroy(bgraph_[m]);
-  }
+  for (int hd = 0; hd < 2; ++hd)
+    for (uint32_t m = 0; m <= kMaxBlock; ++m) {
+      if (bgraph_exec_[hd][m]) (void)hipGraphExecDestroy(bgraph_exec_[hd][m]);
+      if (bgraph_[hd][m]) (void)hipGraphDestroy(bgraph_[hd][m]);
+    }
   if (graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
   if (graph_) (void)hipGraphDestroy(graph_);
   for (void* p : allocs_) (void)hipFree(p);
@@ -298,11 +299,7 @@ bool Engine::init(const uint8_t* b, size_t len, const EngineConfig& cfg, std::st
   build_xm_layouts();  // the gate/up and LM head codes in the matrix-core kernel's load order
   {  // the panels (after everything the decode step reads; CHPE_BLOCK=0: off)
     const char* bk = std::getenv("CHPE_BLOCK");
-    std::string why;
-    if (!(bk && bk[0] == '0') && !plan_panel(&why) && !why.empty()) {
-      *err = "panels: " + why;
-      return false;
-    }
+    if (!(bk && bk[0] == '0')) plan_panel();
   }
   HIP_TRY(hipDeviceSynchronize());
 
@@ -1253,8 +1250,9 @@ uint32_t Engine::enqueue_block_gemv(const ProjPlan* const* parts, float* const* 
   return launch_block_gemv(b, st);
 }
 
-int Engine::block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t* out_argmax, ForwardResult* last) {
-  if (!block_ok_ || !tokens || m == 0 || m > kMaxBlock) return -1;
+int Engine::block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t* out_argmax, ForwardResult* last,
+                          bool head) {
+  if (!block_ok_ || !tokens || m == 0 || m > kMaxBlock || (!head && (out_argmax || last))) return -1;
   if (pos + m > cfg_.max_seq_len) return -2;
   const uint64_t t0 = now_ns();
   const uint32_t mm = uint32_t(m);
@@ -1265,9 +1263,10 @@ int Engine::block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t
       hipMemcpyAsync(d_bstate_, h_bstate_, sizeof(StepState), hipMemcpyHostToDevice, st) != hipSuccess)
     return -3;
   if (cfg_.hybrid && pos == 0) reset_hybrid_state(st);  // a new sequence (outside the graph)
-  if (use_graph_) {  // one captured graph per token count, captured on first use
-    hipGraph_t& g = bgraph_[m];
-    hipGraphExec_t& ge = bgraph_exec_[m];
+  bhead_ = head;
+  if (use_graph_) {  // one captured graph per (head, token count), captured on first use
+    hipGraph_t& g = bgraph_[head ? 1 : 0][m];
+    hipGraphExec_t& ge = bgraph_exec_[head ? 1 : 0][m];
     if (!ge) {
       if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) != hipSuccess) return -3;
       not_built_ = false;
@@ -1289,6 +1288,7 @@ int Engine::block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t
       return -3;
     }
   }
+  if (!head) return hipStreamSynchronize(st) == hipSuccess ? 0 : -3;
   if (hipMemcpyAsync(h_bout_, d_bout_, m * 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
       hipMemcpyAsync(h_result_, d_result_, sizeof(StepResult), hipMemcpyDeviceToHost, st) != hipSuccess)
     return -3;
@@ -1336,6 +1336,7 @@ void Engine::record_block(uint32_t mm, hipStream_t st) {
     const ProjPlan* dn[1] = {&L.down};
     n_ss = enqueue_block_gemv(dn, hid, 1, GemvMode::Accum, d_bmlp_, I, nullptr, 0, mm, l, st);
   }
+  if (!bhead_) return;  // (a prefill block before the last: its logits are not read)
   const ProjPlan* lm[1] = {&lm_head_};
   float* lg[1] = {d_blog_};
   const uint32_t eb = enqueue_block_gemv(lm, lg, 1, GemvMode::Logits, d_bx_, D, d_gamma_final_, n_ss, mm, 0, st);
@@ -1450,6 +1451,7 @@ void Engine::record_block_hybrid(uint32_t mm, hipStream_t st) {
     const ProjPlan* dnp[1] = {&L.down};
     n_ss = enqueue_block_gemv(dnp, hid, 1, GemvMode::Accum, d_bmlp_, I, nullptr, 0, mm, l, st);
   }
+  if (!bhead_) return;  // (a prefill block before the last: its logits are not read)
   const ProjPlan* lm[1] = {&lm_head_};
   float* lg[1] = {d_blog_};
   const uint32_t eb = enqueue_block_gemv(lm, lg, 1, GemvMode::Logits, d_bx_, D, d_gamma_final_, n_ss, mm, 0, st);
@@ -1458,50 +1460,58 @@ void Engine::record_block_hybrid(uint32_t mm, hipStream_t st) {
 }
 
 // ---- panels (a prompt's positions, panel.hip) ---------------------------------------------------
-// Returns false with *err empty when the archive has none (a projection that is neither flat 4- /
-// 2-bit tiles, 4-bit 16-row cells nor fp16 raw tiles), false with *err set on an allocation failure.
-bool Engine::plan_panel(std::string* err) {
+// panel_ok_ stays false when the archive has none (a projection that is neither flat 4- / 2-bit tiles,
+// 4-bit 16-row cells nor fp16 raw tiles), and when their buffers (about 0.6 GB for the 72B model) find no memory
+// or pass CHPE_PANEL_MIB: prompts then run as block steps or decode steps.
+void Engine::plan_panel() {
   panel_ok_ = false;
   const size_t D = arch_.hidden_dim, I = arch_.intermediate_dim;
   const size_t qd = arch_.num_attn_heads * arch_.head_dim, kvd = arch_.num_kv_heads * arch_.head_dim;
   if (!block_ok_) {  // (plan_block's archives have whole plans here; otherwise fp16 raw matrices)
-    if (cfg_.hybrid || D % 128 || I % 128 || qd != D || kvd % 2) return false;
+    if (cfg_.hybrid || D % 128 || I % 128 || qd != D || kvd % 2) return;
     for (const LayerPlan& L : layers_)
       for (const ProjPlan* p : {&L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down})
-        if (p->kind != WeightKind::Raw16 || p->bf16 || size_t(p->rows) * p->cols > (size_t(1) << 30)) return false;
+        if (p->kind != WeightKind::Raw16 || p->bf16 || size_t(p->rows) * p->cols > (size_t(1) << 30)) return;
   }
   auto units = [](size_t rows) { return (rows + 15) / 16; };
   size_t rows_max = std::max({units(qd) + 2 * units(kvd), 2 * units(I), units(D)}) * 16;
   if (cfg_.hybrid) rows_max = std::max<size_t>(rows_max, 8192 + 4096 + 64);
   const size_t Cmax = std::max({D, I, qd}), M = kMaxPanel;
   ppart_floats_ = std::max(2 * rows_max * kPanelRows, size_t(32) << 20);
-  auto fa = [&](size_t n) { return static_cast<float*>(dev_alloc(n * 4)); };
+  const char* mib = std::getenv("CHPE_PANEL_MIB");
+  const size_t first = allocs_.size(), most = mib ? size_t(std::strtoull(mib, nullptr, 10)) << 20 : ~size_t(0);
+  size_t used = 0;
+  bool ok = true;
+  auto bytes = [&](size_t n) -> void* {
+    used += n;
+    void* p = ok && used <= most ? dev_alloc(n) : nullptr;
+    ok = p != nullptr;
+    return p;
+  };
+  auto fa = [&](size_t n) { return static_cast<float*>(bytes(n * 4)); };
   d_px_ = fa(M * D);
   d_pq_ = fa(M * qd);
   d_pattn_ = fa(M * qd);
   d_pmlp_ = fa(M * I);
   // (limbs or three fp16 parts; at most 16 token tiles of kPanelScales scales a group)
-  d_pxs_ = static_cast<uint4*>(dev_alloc(kPanelRows * Cmax * (block_ok_ ? 4 : 6) + 16 * (Cmax / 128) * kPanelScales * 4));
+  d_pxs_ = static_cast<uint4*>(bytes(kPanelRows * Cmax * (block_ok_ ? 4 : 6) + 16 * (Cmax / 128) * kPanelScales * 4));
   d_pxt_ = fa(kPanelRows * Cmax);
   d_ppart_ = fa(ppart_floats_);
   d_pss_ = fa((D + 15) / 16 * M);
-  d_pbrk_ = static_cast<uint32_t*>(dev_alloc(M * 4));
-  d_pstate_ = static_cast<StepState*>(dev_alloc(sizeof(StepState)));
-  bool ok = d_px_ && d_pq_ && d_pattn_ && d_pmlp_ && d_pxs_ && d_pxt_ && d_ppart_ && d_pss_ && d_pbrk_ && d_pstate_;
+  d_pbrk_ = static_cast<uint32_t*>(bytes(M * 4));
+  d_pstate_ = static_cast<StepState*>(bytes(sizeof(StepState)));
   if (cfg_.hybrid) {
     d_phx0_ = fa(M * 8192);
     d_phx1_ = fa(M * 4096);
     d_phx2_ = fa(M * 1024);
     d_phx3_ = fa(M * 32);
     d_phconv_ = fa(M * kDnConvRow);
-    ok = ok && d_phx0_ && d_phx1_ && d_phx2_ && d_phx3_ && d_phconv_;
   }
   if (!ok) {
-    *err = "allocation";
-    return false;
+    for (; allocs_.size() > first; allocs_.pop_back()) (void)hipFree(allocs_.back());
+    (void)hipGetLastError();
   }
-  panel_ok_ = true;
-  return true;
+  panel_ok_ = ok;
 }
 
 uint32_t Engine::enqueue_panel_gemm(const ProjPlan* const* parts, float* const* outs, int n, GemvMode mode,
@@ -1702,9 +1712,12 @@ int Engine::prefill(const uint32_t* tokens, size_t n, ForwardResult* out) {
     h_pos_ = n;
     return 0;
   }
-  uint32_t am[kMaxBlock];  // (n <= kMaxBlock: one block step)
-  const int rc = block_forward(tokens, n, 0, am, out);
-  if (rc) return rc;
+  uint32_t am[kMaxBlock];
+  for (size_t i = 0; i < n; i += kMaxBlock) {  // (past kMaxBlock: no memory for the panels)
+    const size_t m = std::min<size_t>(kMaxBlock, n - i);
+    const bool head = i + m == n;  // (only the last block's logits are read)
+    if (const int rc = block_forward(tokens + i, m, i, head ? am : nullptr, head ? out : nullptr, head)) return rc;
+  }
   // continue greedy decoding from here: the last argmax at position n
   if (set_state(StepState{out->argmax_token, uint32_t(n), 0, 0})) return -3;
   return sync();

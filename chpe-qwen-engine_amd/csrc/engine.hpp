@@ -155,10 +155,12 @@ class Engine {
   // its result *last.  The decode state is not touched.  0, -1 bad arguments or no block step
   // for this archive, -2 past max_seq_len, -3 device error.  (verify() and prefill() then leave
   // the decode state where the sequential steps would: the last argmax at pos + m.)
-  int block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t* out_argmax, ForwardResult* last);
+  // head false: no LM head (out_argmax and last must be null; a prefill's blocks before its last)
+  int block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t* out_argmax, ForwardResult* last,
+                    bool head = true);
   bool block_ready() const { return block_ok_; }
   // positions 0..n-1 teacher-forced: one block step up to kMaxBlock positions, panels
-  // (prompt_forward) above; result and logits of the last position; the decode state is left at
+  // (prompt_forward) above, blocks of kMaxBlock where there is no memory for those; result and logits of the last position; the decode state is left at
   // (argmax of the last, n)
   int prefill(const uint32_t* tokens, size_t n, ForwardResult* out);
   // the prompt in panels of up to kMaxPanel positions (plan_panel's archives; prefill and
@@ -241,7 +243,7 @@ class Engine {
                         const uint32_t* brk, uint32_t m) const;
   DnBlockArgs dn_block_args(size_t l, const float* x0, const float* x1, const float* x2, const float* x3, float* conv,
                             float* out, const uint32_t* brk, uint32_t m) const;
-  bool plan_panel(std::string* err);
+  void plan_panel();
   // m positions pos .. of the prompt (its tokens at d_prompt_ + pos) through every layer
   void enqueue_panel(uint32_t token, uint32_t pos, uint32_t m, hipStream_t st);
   // a panel's projections of one input.  gamma: the rows' n_ss partial sums of squares are in d_pss_,
@@ -324,9 +326,10 @@ class Engine {
   float *d_bhx0_ = nullptr, *d_bhx1_ = nullptr, *d_bhx2_ = nullptr, *d_bhx3_ = nullptr, *d_bhconv_ = nullptr;
   BlockTables btab_{};
   ArgmaxPartial* d_bpartials_ = nullptr;
-  // captured block steps, by token count
-  hipGraph_t bgraph_[kMaxBlock + 1] = {};
-  hipGraphExec_t bgraph_exec_[kMaxBlock + 1] = {};
+  // captured block steps, by [with the LM head][token count]; bhead_: the one being recorded has the LM head
+  hipGraph_t bgraph_[2][kMaxBlock + 1] = {};
+  hipGraphExec_t bgraph_exec_[2][kMaxBlock + 1] = {};
+  bool bhead_ = true;
   // the panels (plan_panel): activations of kMaxPanel rows, the GEMM's input images, partial sums and
   // break flags
   bool panel_ok_ = false;

@@ -212,3 +212,38 @@ def test_refused_launch_is_an_error(w4_archive, call, n):
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("mib", ["0", "40"])
+def test_no_memory_for_panels(w4_archive, mib, monkeypatch):
+    """Where the panels' buffers find no memory (a bound stands for it: none of them, the first few of them) the context
+    still opens, holds none of them, and prompts run as before the panels: chpe_prefill in block steps of up to
+    32 tokens, chpe_forward_tokens past 8 in decode steps, both bit for bit."""
+    import torch
+    toks = np.random.default_rng(9).integers(0, 151936, 75).astype(np.uint32)
+
+    def run(fn):
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        e = ca.Engine(w4_archive, arch=0, max_seq_len=96, kv_f16=False)
+        try:
+            return free - torch.cuda.mem_get_info()[0], fn(e)
+        finally:
+            e.close()
+
+    def steps(e):
+        return [e.decode_step(int(t), p)[1] for p, t in enumerate(toks[:20])][-1]
+
+    def blocks(e):
+        for i in (0, 32, 64):
+            e.verify(toks[i:i + 32], i)
+        return e.logits()
+
+    run(steps)
+    full, want = run(lambda e: (steps(e), blocks(e)))
+    monkeypatch.setenv("CHPE_PANEL_MIB", mib)
+    small, got = run(lambda e: (e.forward_tokens(toks[:20], want_logits=True)[1], e.prefill(toks, want_logits=True)[1]))
+    for a, b in zip(got, want):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    print(f"context: {full >> 20} MiB, without panels {small >> 20}", flush=True)
+    assert small < full - (64 << 20)
