@@ -947,13 +947,18 @@ int Engine::forward_tokens(const uint32_t* toks, size_t n, ForwardResult* out) {
   if (block_ok_ && n > 3 && n <= kSmallBlock) {
     uint32_t am[kSmallBlock];
     if (const int rc = block_forward(toks, n, 0, am, out)) return rc;
+    out->elapsed_ns /= n;  // (a token's, as the last step's below)
     if (set_state(StepState{out->argmax_token, uint32_t(n), 0, 0})) return -3;
     if (hipMemcpyAsync(embed_fused_ ? d_hidden_out_ : d_hidden_, d_bx_ + (n - 1) * arch_.hidden_dim, arch_.hidden_dim * 4,
                        hipMemcpyDeviceToDevice, stream_) != hipSuccess)
       return -3;
     return sync();
   }
-  if (panel_ok_ && n > (block_ok_ ? 3u : 2u)) return prompt_forward(toks, n, out);
+  if (panel_ok_ && n > (block_ok_ ? 3u : 2u)) {
+    const int rc = prompt_forward(toks, n, out);
+    if (rc == 0) out->elapsed_ns /= n;
+    return rc;
+  }
   if (hipMemcpyAsync(d_prompt_, toks, n * 4, hipMemcpyHostToDevice, stream_) != hipSuccess) return -3;
   if (set_state(StepState{toks[0], 0, uint32_t(n), 0})) return -3;
   if (launch_steps(n - 1)) return -3;

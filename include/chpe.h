@@ -30,8 +30,8 @@ void *chpe_init(const char *archive_path);
  * Returns the last argmax, -1 if ctx/tokens is NULL or num_tokens == 0, -2 if num_tokens
  * exceeds the context's max_seq_len, -3 on a device error.  out_logits (optional) receives
  * vocab_size floats of the last step.  More than three positions (two, fp16 raw) run as a block step or
- * in panels where the archive has them (chpe_prefill); chpe_get_last_elapsed_ns is then the whole
- * call's time. */
+ * in panels where the archive has them (chpe_prefill); chpe_get_last_elapsed_ns, the last token's time
+ * in decode steps, is then the call's time over its positions. */
 int chpe_forward_tokens(void *ctx, const uint32_t *tokens, size_t num_tokens, float *out_logits);
 
 /* chpe_c_api.zig:80-87 `chpe_get_last_logits`: copies vocab_size floats of the last step;

@@ -14,6 +14,7 @@ import ctypes
 import os
 import shutil
 import tempfile
+import time
 
 import numpy as np
 import pytest
@@ -247,3 +248,22 @@ def test_no_memory_for_panels(w4_archive, mib, monkeypatch):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
     print(f"context: {full >> 20} MiB, without panels {small >> 20}", flush=True)
     assert small < full - (64 << 20)
+
+
+@pytest.mark.parametrize("n", [3, 6, 40])
+def test_last_elapsed_is_a_tokens(w4_archive, n):
+    """chpe_get_last_elapsed_ns after chpe_forward_tokens is one token's time (chpe_c_api.zig:107-111 after :61-63),
+    whether the positions ran as decode steps, a block step or in panels: n times it is no more than the call,
+    and no less than half of it."""
+    e = ca.Engine(w4_archive, arch=0, max_seq_len=64, kv_f16=False)
+    try:
+        toks = np.random.default_rng(n).integers(0, 151936, n).astype(np.uint32)
+        e.forward_tokens(toks)
+        ratios = []
+        for _ in range(9):
+            t0 = time.perf_counter_ns()
+            e.forward_tokens(toks)
+            ratios.append(n * e.last()["elapsed_ns"] / (time.perf_counter_ns() - t0))
+        assert 0.5 <= sorted(ratios)[4] <= 1.2, ratios
+    finally:
+        e.close()
