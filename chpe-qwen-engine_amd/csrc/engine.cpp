@@ -940,19 +940,13 @@ int Engine::sync() { return hipStreamSynchronize(stream_) == hipSuccess ? 0 : -3
 int Engine::forward_tokens(const uint32_t* toks, size_t n, ForwardResult* out) {
   if (n == 0 || !toks) return -1;
   if (n > cfg_.max_seq_len) return -2;
-  // A few positions: decode steps (the 3B model's three take 3.2 ms, a block step 3.6, a panel 4.6; the 9B
-  // hybrid's 5.3, 3.8, 5.6).  Up to kSmallBlock: the block step.  More: panels (24 positions of the hybrid:
-  // 42 ms as steps, 6.1 as a block step, 5.6 as a panel).  fp16 raw archives, with no block step, take
-  // panels from three positions on (6.3 ms as steps, 4.9).
-  if (block_ok_ && n > 3 && n <= kSmallBlock) {
-    uint32_t am[kSmallBlock];
-    if (const int rc = block_forward(toks, n, 0, am, out)) return rc;
+  // Up to three positions: decode steps (3B: two in 2.4 ms, a block step 3.6).  More: the block step, past
+  // kPromptBlock panels, as prefill does.  fp16 raw archives, with no block step, take panels from three positions on
+  // (6.3 ms as steps, 4.7).
+  if (block_ok_ && n > 3 && n <= kPromptBlock) {
+    if (const int rc = prompt_block(toks, n, out)) return rc;
     out->elapsed_ns /= n;  // (a token's, as the last step's below)
-    if (set_state(StepState{out->argmax_token, uint32_t(n), 0, 0})) return -3;
-    if (hipMemcpyAsync(embed_fused_ ? d_hidden_out_ : d_hidden_, d_bx_ + (n - 1) * arch_.hidden_dim, arch_.hidden_dim * 4,
-                       hipMemcpyDeviceToDevice, stream_) != hipSuccess)
-      return -3;
-    return sync();
+    return 0;
   }
   if (panel_ok_ && n > (block_ok_ ? 3u : 2u)) {
     const int rc = prompt_forward(toks, n, out);
@@ -1707,25 +1701,32 @@ int Engine::prompt_forward(const uint32_t* tokens, size_t n, ForwardResult* out)
   return 0;
 }
 
-int Engine::prefill(const uint32_t* tokens, size_t n, ForwardResult* out) {
-  if (!tokens || n == 0 || !out) return -1;
-  if (n > cfg_.max_seq_len) return -2;
-  if (panel_ok_ && n > kMaxBlock) return prompt_forward(tokens, n, out);  // (a short prompt: the block step's graph)
-  if (!block_ok_) {  // no block step for this archive: sequential steps
-    const int rc = forward_tokens(tokens, n, out);
-    if (rc) return rc;
-    h_pos_ = n;
-    return 0;
-  }
+// a prompt in block steps (past kMaxBlock positions, or past kPromptBlock, only without the panels)
+int Engine::prompt_block(const uint32_t* tokens, size_t n, ForwardResult* out) {
   uint32_t am[kMaxBlock];
-  for (size_t i = 0; i < n; i += kMaxBlock) {  // (past kMaxBlock: no memory for the panels)
-    const size_t m = std::min<size_t>(kMaxBlock, n - i);
+  size_t m = 0;
+  for (size_t i = 0; i < n; i += m) {
+    m = std::min<size_t>(kMaxBlock, n - i);
     const bool head = i + m == n;  // (only the last block's logits are read)
     if (const int rc = block_forward(tokens + i, m, i, head ? am : nullptr, head ? out : nullptr, head)) return rc;
   }
-  // continue greedy decoding from here: the last argmax at position n
+  // continue greedy decoding from here: the last argmax at position n; the last position's hidden state
   if (set_state(StepState{out->argmax_token, uint32_t(n), 0, 0})) return -3;
+  if (hipMemcpyAsync(embed_fused_ ? d_hidden_out_ : d_hidden_, d_bx_ + (m - 1) * arch_.hidden_dim, arch_.hidden_dim * 4,
+                     hipMemcpyDeviceToDevice, stream_) != hipSuccess)
+    return -3;
   return sync();
+}
+
+int Engine::prefill(const uint32_t* tokens, size_t n, ForwardResult* out) {
+  if (!tokens || n == 0 || !out) return -1;
+  if (n > cfg_.max_seq_len) return -2;
+  if (panel_ok_ && n > kPromptBlock) return prompt_forward(tokens, n, out);
+  if (block_ok_) return prompt_block(tokens, n, out);
+  const int rc = forward_tokens(tokens, n, out);  // no block step for this archive
+  if (rc) return rc;
+  h_pos_ = n;
+  return 0;
 }
 
 int Engine::copy_logits(float* out) const {

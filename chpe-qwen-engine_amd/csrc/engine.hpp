@@ -159,7 +159,7 @@ class Engine {
   int block_forward(const uint32_t* tokens, size_t m, size_t pos, uint32_t* out_argmax, ForwardResult* last,
                     bool head = true);
   bool block_ready() const { return block_ok_; }
-  // positions 0..n-1 teacher-forced: one block step up to kMaxBlock positions, panels
+  // positions 0..n-1 teacher-forced: one block step up to kPromptBlock positions, panels
   // (prompt_forward) above, blocks of kMaxBlock where there is no memory for those; result and logits of the last position; the decode state is left at
   // (argmax of the last, n)
   int prefill(const uint32_t* tokens, size_t n, ForwardResult* out);
@@ -167,6 +167,7 @@ class Engine {
   // forward_tokens call it): every weight is read once per panel; result, logits, hidden state and
   // decode state are left as the sequential steps leave them (the last argmax at position n)
   int prompt_forward(const uint32_t* tokens, size_t n, ForwardResult* out);
+  int prompt_block(const uint32_t* tokens, size_t n, ForwardResult* out);  // the same in block steps
   // enqueue n graph launches continuing from the current device state (no sync); -2 and
   // nothing enqueued when the steps would pass max_seq_len
   int launch_steps(size_t n);

@@ -459,6 +459,10 @@ constexpr uint32_t kMaxLogitsBlocks = 8192;
 
 // ---- panels: up to kMaxPanel tokens of a prompt at consecutive positions (panel.hip) ------------
 constexpr uint32_t kMaxPanel = 512;
+// Prompts up to here take the block step, longer ones panels (ms, block step / panel, at 16 and at 20 positions: 3B 4-bit
+// 4.58 / 4.67 and 4.99 / 4.72, 9B hybrid 5.51 / 5.69 and 5.95 / 5.75, 72B 4-bit 26.4 / 26.5 and 28.3 / 26.5; 9B compat
+// 5.67 / 5.42 and 6.12 / 5.47; at 9 positions 4.33 / 4.66, 5.26 / 5.65, 25.5 / 26.4, 5.44 / 5.43)
+constexpr uint32_t kPromptBlock = 16;
 constexpr uint32_t kPanelRows = kMaxPanel + 112;  // rows of the GEMM's buffers: m in whole tiles of up to 112 tokens
 // 16-byte pieces of one 128-column group of a token tile as the GEMM's operands: four limbs of a byte or three
 // fp16 parts, then the tokens' scales (kPanelScales floats, at most 112 of them used: one 4-byte load of 256 lanes)

@@ -81,9 +81,11 @@ int chpe_generate(void *ctx, const uint32_t *prompt, size_t n_prompt, size_t n_g
  * the decode step, bit-identical.  last_* report the final step; chpe_get_last_logits gives
  * its logits.  Returns 0, -1 bad args, -2 pos + m > max_seq_len, -3 device error. */
 int chpe_verify(void *ctx, const uint32_t *drafts, size_t m, size_t pos, uint32_t *out_argmax);
-/* Prefill: positions 0..num_tokens-1 teacher-forced as chpe_forward_tokens: up to 32 positions as
+/* Prefill: positions 0..num_tokens-1 teacher-forced as chpe_forward_tokens: up to 16 positions as
  * one block step, more in panels of up to 512 positions, each reading every weight once (archives of
- * flat 4- or 2-bit tiles, 4-bit 16-row cells or fp16 raw tiles; others: the sequential steps).  Each
+ * flat 4- or 2-bit tiles, 4-bit 16-row cells or, in panels alone, fp16 raw tiles; others: the sequential
+ * steps).  A context whose panel buffers found no device memory, or passed CHPE_PANEL_MIB (MiB, in the
+ * environment at init), runs longer prompts as block steps of up to 32.  Each
  * token's arithmetic is the decode step's up to the order of the float sums; the KV cache holds the
  * same rows.  Leaves the decode state at (the last argmax,
  * num_tokens).  Returns the last argmax, -1 bad args, -2 too long, -3 device error;

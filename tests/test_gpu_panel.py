@@ -220,15 +220,19 @@ def test_no_memory_for_panels(w4_archive, mib, monkeypatch):
     """Where the panels' buffers find no memory (a bound stands for it: none of them, the first few of them) the context
     still opens, holds none of them, and prompts run as before the panels: chpe_prefill in block steps of up to
     32 tokens, chpe_forward_tokens past 8 in decode steps, both bit for bit."""
-    import torch
+    hip = ctypes.CDLL("libamdhip64.so.7")
     toks = np.random.default_rng(9).integers(0, 151936, 75).astype(np.uint32)
 
+    def mem_free():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
     def run(fn):
-        torch.cuda.synchronize()
-        free = torch.cuda.mem_get_info()[0]
+        free = mem_free()
         e = ca.Engine(w4_archive, arch=0, max_seq_len=96, kv_f16=False)
         try:
-            return free - torch.cuda.mem_get_info()[0], fn(e)
+            return free - mem_free(), fn(e)
         finally:
             e.close()
 
@@ -265,5 +269,24 @@ def test_last_elapsed_is_a_tokens(w4_archive, n):
             e.forward_tokens(toks)
             ratios.append(n * e.last()["elapsed_ns"] / (time.perf_counter_ns() - t0))
         assert 0.5 <= sorted(ratios)[4] <= 1.2, ratios
+    finally:
+        e.close()
+
+
+@pytest.mark.parametrize("kind,arch,vocab", [(ca.PACK_3B_W4, 0, 151936), (ca.PACK_3B_FP16_RAW, 0, 151936), (ca.PACK_9B_W4, 3, 248320)])
+def test_both_calls_take_the_same_route(kind, arch, vocab):
+    """chpe_forward_tokens and chpe_prefill of the same tokens give the same bits from four positions on: logits, hidden
+    state and the rows that the next step reads, around each of the rule's edges."""
+    e = ca.Engine(archive_path(kind), arch=arch, max_seq_len=64, kv_f16=True)
+    try:
+        for n in (4, 8, 9, 12, 16, 17, 24, 32, 33):
+            toks = np.random.default_rng(n).integers(0, vocab, n).astype(np.uint32)
+            out = []
+            for call in (e.forward_tokens, e.prefill):
+                am, lg = call(toks, want_logits=True)
+                out.append((am, lg, e.hidden(), e.decode_step(int(toks[0]), n)[1]))
+            assert out[0][0] == out[1][0], n
+            for a, b in zip(out[0][1:], out[1][1:]):
+                assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), n
     finally:
         e.close()
