@@ -8,7 +8,7 @@ Bars as for the other whole-model tests: single-step logits within 2e-4 * max|lo
 >= 0.9999 with the f32 KV cache, 1.5e-3 with the fp16 cache; greedy streams identical, a
 difference allowed only after an oracle step whose top-2 gap is below 1e-3.  Then the state
 machinery: the recurrent states restart at position 0 (a prompt run twice gives the same
-logits bit for bit); the block step (speculative verify of 4 and 8 drafts, the chunked
+logits bit for bit); the block step and the panels (speculative verify of 4, 8 and 32 drafts, the
 prefill: every weight read once, the DeltaNet states rolled over the tokens in order) against
 the decode steps and against the oracle; the hybrid decode is not the reference's decode of the
 same archive (arch 1); the command line's --hybrid writes chpe_forward_tokens' logits of arch
@@ -19,7 +19,7 @@ import pytest
 import chpe_amd as ca
 import oracle as orc
 from test_gpu_cli import receipt, run_cli
-from test_gpu_models import archive, check_stream, compare_logits, say, threads
+from test_gpu_models import archive, check_stream, compare_logits, decode_all, say, threads
 
 pytestmark = pytest.mark.gpu
 
@@ -104,13 +104,13 @@ def test_hybrid_restart_and_block_step(a9h):
         try:
             assert e.block_ready()
             say(f"hybrid kv_f16={kv16}: the prompt twice from position 0")
-            _, l1 = e.forward_tokens(prompt, want_logits=True)
+            l1 = decode_all(e, prompt)
             seq = [e.decode_step(int(d), n + i) for i, d in enumerate(drafts)]
-            _, l2 = e.forward_tokens(prompt, want_logits=True)
+            l2 = decode_all(e, prompt)
             assert np.array_equal(l1.view(np.uint32), l2.view(np.uint32))
             for m in (4, 8):
                 say(f"hybrid: verify {m} drafts vs {m} decode steps")
-                e.forward_tokens(prompt)
+                decode_all(e, prompt)
                 got = e.verify(drafts[:m], n)
                 for i in range(m):
                     if int(got[i]) != int(seq[i][0]):
@@ -119,16 +119,21 @@ def test_hybrid_restart_and_block_step(a9h):
                 if m == 4:  # the decode state continues after the block: the next draft's step
                     am, lg = e.decode_step(int(drafts[4]), n + 4)
                     compare_logits(lg, seq[4][1], "decode step after verify 4", rel)
-            say("hybrid: prefill (a block step of 6) vs forward_tokens")
+            say("hybrid: prefill (a block step of 6) vs decode steps")
             _, lp = e.prefill(prompt, want_logits=True)
-            compare_logits(lp, l1, "prefill vs forward_tokens", rel)
+            compare_logits(lp, l1, "prefill vs decode steps", rel)
             am, lg = e.decode_step(int(drafts[0]), n)
             compare_logits(lg, seq[0][1], "decode step after prefill", rel)
-            say("hybrid: prefill of 40 positions (blocks of 32 + 8) vs forward_tokens")
-            long = prompt_of(13, 40)
-            _, ls = e.forward_tokens(long, want_logits=True)
+            say("hybrid: prefill of 40 positions (a panel) and a verify of 32 vs decode steps")
+            long, many = prompt_of(13, 40), prompt_of(14, 32)
+            ls = decode_all(e, long)
             _, lb = e.prefill(long, want_logits=True)
-            compare_logits(lb, ls, "prefill 40 vs forward_tokens", rel)
+            compare_logits(lb, ls, "prefill 40 vs decode steps", rel)
+            decode_all(e, prompt)
+            lm = [e.decode_step(int(d), n + i)[1] for i, d in enumerate(many)][-1]
+            decode_all(e, prompt)
+            e.verify(many, n)
+            compare_logits(e.logits(), lm, "verify 32: last draft", rel)
             if kv16:
                 # a step at position 1 continues from the state position 0 left
                 a = e.decode_step(int(prompt[0]), 0)[1]

@@ -145,13 +145,18 @@ def top2_gap(lg):
     return float(t[-1] - t[-2])
 
 
+def decode_all(e, tokens):
+    """the last position's logits after a decode step per position"""
+    return [e.decode_step(int(t), p)[1] for p, t in enumerate(tokens)][-1]
+
+
 def run_block(path, arch, vocab, seed, oracle_check, block=True):
-    """The block step (every weight read once for up to 32 tokens; no reference code, defined as
-    the decode steps it replaces) against the decode step on the same engine: chpe_prefill vs
-    chpe_forward_tokens (the last position's logits, then one decode step on each cache, so the
-    KV rows agree; 11 tokens: one block of the 512-column ranges with 3 token quads; 43 tokens:
-    a full block of 32 and one of 11), chpe_verify of 8 drafts vs 8 decode steps (every argmax,
-    the last logits; the 2048-column ranges).
+    """The block step (every weight read once for up to 32 tokens) and the panels (up to 512), which have no
+    reference code and are defined as the decode steps they replace, against decode steps, one call a
+    position, on the same engine: chpe_prefill (the last position's logits, then one decode step on each cache, so the
+    KV rows agree; 11 tokens: one block of the 512-column ranges with 3 token quads; 17, 43, 70, 90 and 105: panels
+    with token tiles of 32, 64, 80, 96 and, on the 72B archives, 112), chpe_verify of 8 and of 32 drafts vs as many decode
+    steps (every argmax, the last logits; the 2048-column ranges, the output-stationary GEMM).
     Bars: 2e-4 * max|logit| with the f32 cache, as for the decode step against the oracle;
     3e-3 with the fp16 cache, twice the single-step bar: the two paths sum in different orders,
     so k / v elements near an fp16 rounding boundary round differently, and here 19 cached
@@ -164,7 +169,7 @@ def run_block(path, arch, vocab, seed, oracle_check, block=True):
     drafts = rng.integers(0, vocab, 8).astype(np.uint32)
     n = len(prompt)
     for kv16, rel in ((False, 2e-4), (True, 3e-3)):
-        e = ca.Engine(path, arch=arch, max_seq_len=64, kv_f16=kv16)
+        e = ca.Engine(path, arch=arch, max_seq_len=128, kv_f16=kv16)
         try:
             assert e.block_ready() == block
             if not e.block_ready():  # no block step: prefill and verify are the decode steps, bit for bit
@@ -175,26 +180,35 @@ def run_block(path, arch, vocab, seed, oracle_check, block=True):
                 assert list(e.verify(drafts[:4], n)) == seq
                 continue
             say(f"block step arch {arch} kv_f16={kv16}: sequential reference")
-            _, lseq = e.forward_tokens(prompt, want_logits=True)
+            lseq = decode_all(e, prompt)
             seq = [e.decode_step(int(d), n + i) for i, d in enumerate(drafts)]
             say("  prefill of 11 positions (one block)")
             _, lblk = e.prefill(prompt, want_logits=True)
-            compare_logits(lblk, lseq, "prefill vs forward_tokens", rel)
+            compare_logits(lblk, lseq, "prefill vs decode steps", rel)
             am, lg = e.decode_step(int(drafts[0]), n)
             compare_logits(lg, seq[0][1], "decode step after prefill", rel)
-            say("  prefill of 43 positions (a block of 32 + 11) vs forward_tokens")
-            long = rng.integers(0, vocab, 43).astype(np.uint32)
-            _, lseq2 = e.forward_tokens(long, want_logits=True)
-            _, lblk2 = e.prefill(long, want_logits=True)
-            compare_logits(lblk2, lseq2, "prefill 43 vs forward_tokens", rel)
-            e.forward_tokens(prompt)  # (the context of the verify below)
-            say("  verify 8 drafts")
-            got = e.verify(drafts, n)
-            for i in range(8):
-                ref_am, ref_lg = seq[i]
-                if got[i] != ref_am:
-                    assert top2_gap(ref_lg) < 2 * rel * float(np.abs(ref_lg).max()), (i, int(got[i]), int(ref_am))
-            compare_logits(e.logits(), seq[7][1], "verify: last draft", rel)
+            for k in (17, 43, 70, 90, 105):
+                say(f"  prefill of {k} positions (a panel) vs decode steps")
+                long = rng.integers(0, vocab, k).astype(np.uint32)
+                lseq2 = decode_all(e, long)
+                nseq2 = e.decode_step(int(drafts[0]), k)[1]
+                _, lblk2 = e.prefill(long, want_logits=True)
+                compare_logits(lblk2, lseq2, f"prefill {k} vs decode steps", rel)
+                compare_logits(e.decode_step(int(drafts[0]), k)[1], nseq2, f"decode step after prefill {k}", rel)
+
+            def check_verify(tokens, ref):
+                got = e.verify(tokens, n)
+                for i, (ref_am, ref_lg) in enumerate(ref):
+                    if got[i] != ref_am:
+                        assert top2_gap(ref_lg) < 2 * rel * float(np.abs(ref_lg).max()), (i, int(got[i]), int(ref_am))
+                compare_logits(e.logits(), ref[-1][1], f"verify {len(tokens)}: last draft", rel)
+
+            many = rng.integers(0, vocab, 32).astype(np.uint32)
+            decode_all(e, prompt)  # (the context of the verifies below)
+            ref32 = [e.decode_step(int(d), n + i) for i, d in enumerate(many)]
+            say("  verify 32 and 8 drafts")
+            check_verify(many, ref32)
+            check_verify(drafts, seq)
             if oracle_check and not kv16:
                 o = orc.Oracle(path, arch=arch, max_seq_len=64, kv_f16=False, threads=threads())
                 try:

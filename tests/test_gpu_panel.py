@@ -2,14 +2,13 @@
 steps of an engine that has neither (CHPE_BLOCK=0): the last position's logits and hidden state, and
 the next decode step's logits, which read every cache row and recurrent state the panels left.
 
-Prompt lengths at the edges of the block step (4, 8), of the token tiles (32, 64), of the DeltaNet chunk (32) and of the panel
-(512), and odd ones.  The 2-norm bars: with the f32 cache each path is within 1e-5 of the 64-bit
+Prompt lengths at the edges of the block step (4, 8, 16), of the token tiles (32, 64, and 90 and 200 for those of
+96 and 112), of the DeltaNet chunk (32) and of the panel (512), and odd ones.  The 2-norm bars: with the f32 cache each path is within 1e-5 of the 64-bit
 result (f32 sums over 36 layers; measured 1e-6 to 8e-6), so they differ by less than 2e-5, with as
 much again for the prompt; with the fp16 cache, rows whose f32 value lies within that distance of a
 rounding boundary are stored one fp16 step apart (2^-11 of the value): measured 1e-5 to 2e-4, the
 bars four times that.  An argmax may differ only where the two best logits are closer
-than the bar.  (The 72B archives' panels: test_gpu_models.py, a prompt of 11 against the block step
-and the oracle.)"""
+than the bar.  (The 72B archives' panels: test_gpu_models.py, every tile against decode steps.)"""
 import ctypes
 import os
 import shutil
@@ -26,11 +25,11 @@ from conftest import archive_path
 pytestmark = pytest.mark.gpu
 
 CASES = [  # archive kind, arch, vocabulary, fp16 cache, prompt lengths, bar
-    (ca.PACK_3B_W4, 0, 151936, False, (4, 8, 9, 32, 33, 64, 65, 129, 512, 513, 577), 4e-5),
+    (ca.PACK_3B_W4, 0, 151936, False, (4, 8, 9, 16, 17, 32, 33, 64, 65, 90, 129, 200, 512, 513, 577), 4e-5),
     (ca.PACK_3B_W4, 0, 151936, True, (5, 97, 600), 8e-4),
     (ca.PACK_3B_FP16_RAW, 0, 151936, False, (3, 31, 33, 64, 100, 515), 4e-5),
     (ca.PACK_3B_FP16_RAW, 0, 151936, True, (7, 130), 8e-4),
-    (ca.PACK_9B_W4, 3, 248320, True, (4, 9, 32, 33, 65, 100, 513), 8e-4),
+    (ca.PACK_9B_W4, 3, 248320, True, (4, 9, 16, 17, 32, 33, 65, 90, 100, 200, 513), 8e-4),
     (ca.PACK_9B_W4, 3, 248320, False, (5, 70), 8e-5),
     (ca.PACK_9B_W4, 1, 248320, False, (34, 70), 8e-5),
 ]
@@ -58,7 +57,10 @@ def test_panels_match_decode_steps(kind, arch, vocab, kv16, lengths, bar, monkey
             am0, want = steps.forward_tokens(toks, want_logits=True)
             hid0 = steps.hidden()
             nxt0 = steps.decode_step(int(toks[0]), n)[1]
-            calls = [e.forward_tokens] + ([e.prefill] if n > 32 else [])
+            steps.forward_tokens(toks)
+            steps.time_steps(1)  # (the greedy loop's next step, from the device state the prompt left)
+            gen0 = steps.logits()
+            calls = [e.forward_tokens] + ([e.prefill] if n > 16 else [])
             for call in calls:
                 am, got = call(toks, want_logits=True)
                 hid = e.hidden()
@@ -69,9 +71,10 @@ def test_panels_match_decode_steps(kind, arch, vocab, kv16, lengths, bar, monkey
                 assert max(d) <= bar
                 if am != am0:
                     assert want[am0] - want[am] <= bar * np.linalg.norm(want)
-            # the greedy loop goes on from the state the prompt left
-            assert np.array_equal(e.forward_tokens(toks, want_logits=True)[1].view(np.uint32),
-                                  e.forward_tokens(toks, want_logits=True)[1].view(np.uint32))
+                    continue
+                assert np.array_equal(call(toks, want_logits=True)[1].view(np.uint32), got.view(np.uint32))
+                e.time_steps(1)
+                assert rel(e.logits(), gen0) <= bar
     finally:
         e.close()
         steps.close()

@@ -49,3 +49,15 @@ def test_launchers_refuse_what_is_not_built():
     dn = lib._ZN4chpe15launch_dn_blockERKNS_11DnBlockArgsEP12ihipStream_t
     dn.restype, dn.argtypes = ctypes.c_bool, [ctypes.c_void_p, ctypes.c_void_p]
     assert dn(args, None) is False
+
+
+def test_gpu_lengths_reach_every_tile():
+    """The prompt lengths of the GPU tests take every token tile, on the 72B launches (test_gpu_models.py, both code widths)
+    and on the 3B and 9B ones (test_gpu_panel.py)."""
+    def tiles(launches, lengths):
+        room = max(2 * max(u for u, _ in launches) * 16 * (PANEL + 112), 32 << 20)
+        return {shape(u, g, m, b, room).tile for u, g in launches for m in lengths for b in (2, 4)}
+
+    assert tiles([(640, 64), (512, 64), (3696, 64), (512, 231)], (17, 43, 70, 90, 105)) == set(TILES[4])
+    assert tiles([(160, 16), (128, 16), (1376, 16), (128, 86)], (17, 32, 33, 64, 65, 90, 129, 200)) == set(TILES[4])
+    assert tiles([(772, 32), (640, 32), (256, 32), (1536, 32), (256, 96)], (17, 32, 33, 65, 90, 100, 200)) == set(TILES[4])
