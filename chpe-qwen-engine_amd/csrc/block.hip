@@ -1,6 +1,6 @@
 // block.hip -- the block step's GEMV: m <= kMaxBlock tokens at consecutive positions through
 // flat 4- or 2-bit tiles (gemvCellFlat, chpe_engine.zig:584-729), every weight read once for all
-// of them.  Used by the batch-M verify and by prompts of up to 32 positions; each token's arithmetic is the
+// of them.  Used by the batch-M verify and by short prompts (kPromptBlock); each token's arithmetic is the
 // batch-1 step's (forwardDecode :1663-1803).
 //
 // 1. k_block_limbs: per token the GEMV input (RMS-normalised, (x * inv) * gamma, rmsNorm

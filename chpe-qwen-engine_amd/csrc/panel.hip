@@ -550,7 +550,7 @@ __global__ void __launch_bounds__(256, 2) k_panel_gemm_h(PanelGemmArgs a) {
 // The ranges' sums of the OPW rows in flight together; then the rows' packed correction entries,
 // which are one consecutive run: 64 entries in one load, one per lane, and 16 columns' loads in
 // flight at a time, whatever row they belong to (row by row, with an entry load and a column load
-// chain each, the SwiGLU launch of the 72B model at 300 tokens took 334 us; this way EPI_US).  Then
+// chain each, the SwiGLU launch of the 72B model at 300 tokens took 334 us; this way 92).  Then
 // through LDS to outputs-fastest order for the writes.  Bound by the corrections' reads (4 bytes
 // per entry and token, from L2) and the partial sums.
 template <int MODE, int OPW>
