@@ -1172,7 +1172,7 @@ bool Engine::plan_packed_corrections(const std::vector<float2>& padded, size_t r
   pk.reserve(padded.size());
   for (size_t r = 0; r < rows; ++r) {
     off[r] = uint32_t(pk.size());
-    for (uint32_t k = 0; k < kmax; ++k) {
+    for (uint32_t k = 0; k < kmax && r * kmax + k < padded.size(); ++k) {  // (a short tensor's table ends at its last row)
       const float2 e = padded[r * kmax + k];
       if (e.y != 0.0f) pk.push_back(e);  // (a NaN weight stays: it makes the row NaN)
     }
